@@ -105,6 +105,19 @@ int stk_speculate(const void* q, const void* k, const void* v, int dtype, int hq
                   float* low_l, float* low_u, float* low_abs, void* retained_ids,
                   uint8_t* overflow, float* mass_m, float* mass_l, void* stream);
 
+/* strict_topk/kernels.py:480-501 speculate in compact mode, with scratch
+ * memory: outputs as above.  The workspace size is 0, and the call is
+ * stk_speculate(mode = 2), for shapes without a scratch-memory form (FP32,
+ * D outside {64, 128, 256}, B not a multiple of 16, s > 256, or operands
+ * not 16-byte aligned). */
+size_t stk_compact_workspace_bytes(int dtype, int hq, int b, int d, int s);
+int stk_speculate_compact(const void* q, const void* k, const void* v, int dtype, int hq, int hkv,
+                          int n, int b, int d, const void* pred, int pred_dtype, int s, float tau,
+                          int capacity, float* m, float* l, float* u, uint8_t* high, float* low_m,
+                          float* low_l, float* low_u, float* low_abs, void* retained_ids,
+                          uint8_t* overflow, float* mass_m, float* mass_l, void* workspace,
+                          size_t workspace_bytes, void* stream);
+
 /* strict_topk/kernels.py:553-560 touch_kv: per (head, slot, 1024-element
  * tile) sum of K + V of the predicted block, out[H,S,ceil(B*D/1024)]. */
 int stk_touch_kv(const void* k, const void* v, int dtype, int h, int n, int b, int d,

@@ -157,7 +157,10 @@ struct TokTile {
         float alpha = wexp(m, nm);
         l *= alpha;
 #pragma unroll
-        for (int e = 0; e < DPL; ++e) acc[e] *= alpha;
+        for (int e = 0; e < DPL; ++e) {
+          acc[e] *= alpha;
+          if constexpr (ABS) aacc[e] *= alpha;
+        }
         m = nm;
       }
     }
@@ -268,23 +271,26 @@ struct TokTileW : TokTile<T, NCH, UP> {
   // Online softmax over one chunk (token t0 + j valid when < Bn).  MASKV:
   // the tokens at or past Bn hold no data and their values are taken as
   // zero (a partly filled block; whatever the memory holds adds nothing).
-  template <bool MASKV = false>
+  // FIXED keeps m as the exponent frame (no rescaling).
+  template <bool MASKV = false, bool FIXED = false>
   __device__ __forceinline__ void update(const uint32_t* qw, const uint32_t (&kw)[UP][QW],
                                          const uint4 (&vw)[NV], int t0, int Bn, float scale,
                                          float& m, float& l, float (&acc)[ACC]) const {
     float s[UP];
     this->scores(qw, kw, t0, Bn, scale, s);
-    float cm = s[0];
+    if constexpr (!FIXED) {
+      float cm = s[0];
 #pragma unroll
-    for (int u = 1; u < UP; ++u) cm = fmaxf(cm, s[u]);
-    cm = wave_max_u(cm);
-    const float nm = fmaxf(m, cm);
-    if (nm > m) {
-      const float alpha = wexp(m, nm);
-      l *= alpha;
+      for (int u = 1; u < UP; ++u) cm = fmaxf(cm, s[u]);
+      cm = wave_max_u(cm);
+      const float nm = fmaxf(m, cm);
+      if (nm > m) {
+        const float alpha = wexp(m, nm);
+        l *= alpha;
 #pragma unroll
-      for (int e = 0; e < ACC; ++e) acc[e] *= alpha;
-      m = nm;
+        for (int e = 0; e < ACC; ++e) acc[e] *= alpha;
+        m = nm;
+      }
     }
     float w[UP], ws = 0.f;
 #pragma unroll

@@ -37,6 +37,9 @@ _SIGS = {
     "stk_exact_attention": (I, [P, P, P, I, I, I, I, I, I, P, I, I, P, P, Z, P]),
     "stk_speculate": (I, [P, P, P, I, I, I, I, I, I, P, I, I, I, F, I,
                           P, P, P, P, P, P, P, P, P, P, P, P, P]),
+    "stk_compact_workspace_bytes": (Z, [I, I, I, I, I]),
+    "stk_speculate_compact": (I, [P, P, P, I, I, I, I, I, I, P, I, I, F, I,
+                                  P, P, P, P, P, P, P, P, P, P, P, P, P, Z, P]),
     "stk_touch_kv": (I, [P, P, I, I, I, I, I, P, I, I, P, P]),
     "stk_fallback": (I, [P, P, P, I, I, I, I, I, I, P, I, I, P, P, P]),
     "stk_repair_workspace_bytes": (Z, [I, I, I, I, I, I]),

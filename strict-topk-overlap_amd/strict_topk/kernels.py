@@ -152,11 +152,14 @@ def speculate(q, k, v, predicted, mode='saved', mass_threshold=0.1, *, keep_mass
         high = torch.empty((h, s), device=dev, dtype=torch.bool)
         retained_ids = torch.empty((h, c), device=dev, dtype=predicted.dtype)
         overflow = torch.empty((h,), device=dev, dtype=torch.bool)
-        _lib.call("stk_speculate", *_args(q, k, v), _lib.ptr(predicted), _lib.id_code(predicted),
-                  s, 2, float(mass_threshold), c, _lib.ptr(state.m), _lib.ptr(state.l),
-                  _lib.ptr(state.u), _lib.ptr(high), _lib.ptr(low.m), _lib.ptr(low.l),
-                  _lib.ptr(low.u), _lib.ptr(low_abs), _lib.ptr(retained_ids), _lib.ptr(overflow),
-                  _lib.ptr(pm), _lib.ptr(pl), _lib.stream(dev))
+        nbytes = _lib.size("stk_compact_workspace_bytes", _lib.dtype_code(q), h, b, d, s)
+        ws = _lib.workspace(nbytes, dev) if nbytes else None
+        _lib.call("stk_speculate_compact", *_args(q, k, v), _lib.ptr(predicted),
+                  _lib.id_code(predicted), s, float(mass_threshold), c, _lib.ptr(state.m),
+                  _lib.ptr(state.l), _lib.ptr(state.u), _lib.ptr(high), _lib.ptr(low.m),
+                  _lib.ptr(low.l), _lib.ptr(low.u), _lib.ptr(low_abs), _lib.ptr(retained_ids),
+                  _lib.ptr(overflow), _lib.ptr(pm), _lib.ptr(pl), _lib.ptr(ws), nbytes,
+                  _lib.stream(dev))
         mass_m, mass_l = (pm, pl) if keep_mass else (None, None)
         return Prediction(state, 'compact', high, low, retained_ids, overflow, low_abs, mass_m, mass_l)
     state = _allocate_state(h, s, d, dev)
