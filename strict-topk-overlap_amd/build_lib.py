@@ -23,7 +23,7 @@ BUILD = ROOT / "_build"
 ARCH = "gfx950"
 SOURCES = ["api.cpp", "states.hip", "select.hip", "repair.hip", "signed.hip", "hier.hip", "sstep.hip",
            "bounds.hip", "indexer.hip", "paged.hip", "step.hip", "tail_dense.hip", "front_pg.hip",
-           "tail_pg.hip", "stail_pg.hip", "cache.hip", "srepair.hip", "compact.hip",
+           "tail_pg.hip", "stail_pg.hip", "cache.hip", "srepair.hip", "srepair_compact.hip", "compact.hip",
            "hier_mfma.hip", "step1.hip", "repair_fast.hip", "step_small.hip"]
 
 FLAGS = [

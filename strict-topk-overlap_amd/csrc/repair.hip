@@ -12,6 +12,7 @@
 // LDS reductions.  Query head h reads KV head h / (Hq / Hkv).
 #include "gqa_repair.hpp"
 #include "repair_fast.hpp"
+#include "srepair.hpp"
 #include "api.hpp"
 
 namespace stk {
@@ -449,6 +450,16 @@ STK_API int stk_repair(const void* q, const void* k, const void* v, int dtype, i
   STK_REQUIRE(workspace && workspace_bytes >= stk_repair_workspace_bytes(hq, sa, sp, sc, d, mode),
               "workspace too small");
   hipStream_t st = (hipStream_t)stream;
+  const uintptr_t align = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
+                          reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(pu);
+  if ((mode == MODE_COMPACT || sc == sp) && srepair_covers(dtype, b, d, sa, sp, sc, align)) {
+    SRepairArgs r{{q, k, v, hq, hkv, n, b, d}, selected, sel_dtype, sa, predicted, pred_dtype, sp,
+                  mode != MODE_SAVED ? 1 : 0, sc, mode == MODE_COMPACT ? retained_ids : nullptr, 1,
+                  pm, pl, pu, high, low_m, low_l, low_u, low_abs, nullptr, nullptr, min_remaining,
+                  cancellation_tol, 0.f, nullptr, 0, 0, nullptr, nullptr, out, fallback, remaining,
+                  nullptr, nullptr};
+    return launch_srepair(dtype, r, st);
+  }
   Carve w(workspace);
   uint8_t* hit = w.take<uint8_t>((size_t)hq * sc);
   uint8_t* miss = w.take<uint8_t>((size_t)hq * sa);
@@ -524,6 +535,17 @@ STK_API int stk_repair_fused(const void* q, const void* k, const void* v, int dt
   STK_REQUIRE(max_extra_mass == 0.f || (approximate && extra_mass_bound), "null budget outputs");
   STK_REQUIRE(max_extra_mass == 0.f || mode == MODE_SAVED || (mass_m && mass_l),
               "positive max_extra_mass requires speculate(..., keep_mass=True)");
+  hipStream_t st = (hipStream_t)stream;
+  const uintptr_t align = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
+                          reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(pu);
+  if ((mode == MODE_COMPACT || sc == sp) && srepair_covers(dtype, b, d, sa, sp, sc, align)) {
+    SRepairArgs r{{q, k, v, hq, hkv, n, b, d}, selected, sel_dtype, sa, predicted, pred_dtype, sp,
+                  mode != MODE_SAVED ? 1 : 0, sc, mode == MODE_COMPACT ? retained_ids : nullptr, 0,
+                  pm, pl, pu, high, low_m, low_l, low_u, low_abs, mass_m, mass_l, min_remaining,
+                  cancellation_tol, max_extra_mass, nullptr, 0, 0, nullptr, nullptr, out, fallback,
+                  remaining, approximate, extra_mass_bound};
+    return launch_srepair(dtype, r, st);
+  }
   FusedArgs f{};
   f.kv = KV{q, k, v, hq, hkv, n, b, d};
   f.a = selected; f.atype = sel_dtype; f.sa = sa;
@@ -533,7 +555,6 @@ STK_API int stk_repair_fused(const void* q, const void* k, const void* v, int dt
   f.min_remain = min_remaining; f.cancel = cancellation_tol; f.eps = max_extra_mass;
   f.out = out; f.bad = fallback; f.remain = remaining; f.approx = approximate;
   f.extra = extra_mass_bound;
-  hipStream_t st = (hipStream_t)stream;
   STK_DISPATCH_TILE(dtype, d, {
     hipLaunchKernelGGL((k_repair_fused<T, VEC, NC, U>), dim3(hq), dim3(256), 0, st, f);
   });
