@@ -299,7 +299,7 @@ STK_API int stk_cache_step(const void* q, int dtype, int requests, int hq, int h
   uint64_t* keys = static_cast<uint64_t*>(workspace);
   const int pages = R * hkv * slots_per_group;
   FrontArgs f = make_front_args(q, k_slots, v_slots, dtype, hqa, hkva, nb, b, d, lo_pages,
-                                hi_pages, bounds_dtype != 0, predicted, sp, m, l, u, keys, s);
+                                hi_pages, bounds_dtype != 0, predicted, sp, m, l, u, keys, s, true);
   f.pg = Paging{table, nblocks, hkv, pages, ntokens, host_table, host_pages};
   hipStream_t st = (hipStream_t)stream;
   int rc = launch_front_pg(dtype, f, s, st);

@@ -30,6 +30,8 @@
 
 #include "attn.hpp"
 
+#include <type_traits>
+
 namespace stk {
 
 constexpr int kScoreWaves = 4;
@@ -353,6 +355,147 @@ __device__ __forceinline__ void score_wg(const ScoreArgs& a, int wg,
       st_agent(a.sflag + (size_t)(h0 + threadIdx.x) * a.fstride + chunk,
                ((mx >> 16) << 16) | (mn >> 16));
     }
+  }
+}
+
+// Scoring workgroup of a large grid (4 waves; FULL shapes, no flags): chunks
+// first .. first + cpw - 1 of KV row kv, the next chunk's bounds requested (PG:
+// the one after's table entries too) before this one's arithmetic, the query
+// values of all G <= GM heads staged once.  The sums are those of score_wg, bit
+// for bit.  Chunks past the row's blocks are skipped.
+template <typename Q, int P, int STEPS, int GT, int GM, bool PG>
+__device__ __forceinline__ void score_wg_multi(const ScoreArgs& a, int kv, int first,
+                                               int cpw, const Paging& pg = Paging{}) {
+  constexpr int C = GT * STEPS;
+  constexpr int BPC = kScoreWaves * 4 * STEPS;   // blocks per chunk
+  __shared__ __align__(16) double s_q[GM * 64 * P];
+  __shared__ __align__(16) uint32_t s_m[GM * 64 * P];
+  const int G = a.hq / a.hkv;
+  const int nv = PG ? pg_blocks(pg, kv, a.n) : a.n;
+  if (first * BPC >= nv) return;
+  const int h0 = kv * G;
+  const int lane = lane_id(), l16 = lane & 15, c = score_lane(l16), sub = lane >> 4;
+  const int wbase = wave_id() * (4 * STEPS);
+  int last = (nv - 1) / BPC;
+  if (last > first + cpw - 1) last = first + cpw - 1;
+  // bounds rows of chunk x (past the last chunk: the last one's again)
+  auto pages = [&](int x, int (&row)[STEPS]) {
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      const int nb = (x < last ? x : last) * BPC + wbase + 4 * s + sub;
+      if constexpr (PG) row[s] = pg_bounds_row(pg, kv, a.n, nb, nb < nv);
+      else row[s] = nb < nv ? nb : -1;
+    }
+  };
+  const size_t base = PG ? 0 : (size_t)kv * a.n;
+  auto body = [&](auto wide) {
+    // W: 32-bit words per lane and pass: 2 (16-bit bounds) or 4 (FP32)
+    constexpr int W = decltype(wide)::value;
+    auto fetch = [&](const int (&row)[STEPS], uint32_t (&lw)[STEPS][P][W],
+                     uint32_t (&hw)[STEPS][P][W]) {
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s) {
+        const size_t r = (base + (size_t)(row[s] < 0 ? 0 : row[s])) * a.d;
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+          const size_t o = r + 64 * j + 4 * c;
+          if constexpr (W == 2) {
+            const uint2 x = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(a.lo) + o);
+            const uint2 y = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(a.hi) + o);
+            lw[s][j][0] = x.x; lw[s][j][1] = x.y;
+            hw[s][j][0] = y.x; hw[s][j][1] = y.y;
+          } else {
+            const uint4 x = *reinterpret_cast<const uint4*>(static_cast<const float*>(a.lo) + o);
+            const uint4 y = *reinterpret_cast<const uint4*>(static_cast<const float*>(a.hi) + o);
+            lw[s][j][0] = x.x; lw[s][j][1] = x.y; lw[s][j][2] = x.z; lw[s][j][3] = x.w;
+            hw[s][j][0] = y.x; hw[s][j][1] = y.y; hw[s][j][2] = y.z; hw[s][j][3] = y.w;
+          }
+        }
+      }
+    };
+    auto widen = [&](const uint32_t (&w)[W], float (&f)[4]) {
+      if constexpr (W == 2) {
+        Unpack<Q>::run(w[0], f);
+        Unpack<Q>::run(w[1], f + 2);
+      } else {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) f[t] = __uint_as_float(w[t]);
+      }
+    };
+    auto score = [&](int x, const int (&row)[STEPS], const uint32_t (&lw)[STEPS][P][W],
+                     const uint32_t (&hw)[STEPS][P][W]) {
+      for (int gb = 0; gb < G; gb += GT) {
+        double acc[C];
+#pragma unroll
+        for (int i = 0; i < C; ++i) acc[i] = 0.0;
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+          float lf[STEPS][4], hf[STEPS][4];
+#pragma unroll
+          for (int s = 0; s < STEPS; ++s) {
+            widen(lw[s][j], lf[s]);
+            widen(hw[s][j], hf[s]);
+          }
+#pragma unroll
+          for (int gi = 0; gi < GT; ++gi) {
+            const int x0 = (gb + gi) * 64 * P + 64 * j + 4 * c;
+            const double2 q01 = *reinterpret_cast<const double2*>(s_q + x0);
+            const double2 q23 = *reinterpret_cast<const double2*>(s_q + x0 + 2);
+            const uint4 mk = *reinterpret_cast<const uint4*>(s_m + x0);
+            const double qd[4] = {q01.x, q01.y, q23.x, q23.y};
+            const uint32_t mm[4] = {mk.x, mk.y, mk.z, mk.w};
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+              for (int t = 0; t < 4; ++t) {
+                const uint32_t bits = (__float_as_uint(lf[s][t]) & mm[t]) |
+                                      (__float_as_uint(hf[s][t]) & ~mm[t]);
+                acc[gi * STEPS + s] =
+                    fma(qd[t], (double)__uint_as_float(bits), acc[gi * STEPS + s]);
+              }
+          }
+        }
+        double r = score_rowsum<C>(acc, l16);
+        constexpr int LOGC = C == 8 ? 3 : (C == 4 ? 2 : (C == 2 ? 1 : 0));
+        const int combo = l16 >> (4 - LOGC);
+        const int gi = combo / STEPS, s = combo % STEPS;
+        const int nb = x * BPC + wbase + 4 * s + sub;
+        bool dead = false;
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) dead = i == s ? row[i] < 0 : dead;
+        const bool mine = (l16 & ((16 >> LOGC) - 1)) == 0 && nb < nv && gb + gi < G;
+        if (r == 0.0) r = 0.0;
+        if (mine) a.keys[(size_t)(h0 + gb + gi) * a.n + nb] = PG && dead ? 0ull : score_key(r);
+      }
+    };
+    int ra[STEPS], rb[STEPS];
+    uint32_t la[STEPS][P][W], ha[STEPS][P][W], lb[STEPS][P][W], hb[STEPS][P][W];
+    pages(first, ra);
+    pages(first + 1, rb);
+    fetch(ra, la, ha);
+    const Q* qbase = reinterpret_cast<const Q*>(a.q) + (size_t)h0 * a.d;
+    for (int x = threadIdx.x; x < GM * 64 * P; x += kScoreWaves * STK_WAVE) {
+      const float qv = x < G * 64 * P ? cvt(qbase[x]) : 0.f;   // d == 64 P
+      s_q[x] = (double)qv;
+      s_m[x] = qv >= 0.f ? 0u : ~0u;   // lo where q < 0 or q is NaN
+    }
+    __syncthreads();
+    for (int x = first; x <= last; x += 2) {
+      int rn[STEPS];
+      fetch(rb, lb, hb);
+      pages(x + 2, rn);
+      score(x, ra, la, ha);
+      if (x + 1 > last) break;
+      fetch(rn, la, ha);
+#pragma unroll
+      for (int s = 0; s < STEPS; ++s) ra[s] = rn[s];
+      score(x + 1, rb, lb, hb);
+      pages(x + 3, rb);
+    }
+  };
+  if constexpr (sizeof(Q) == 2) {
+    if (a.lb) body(std::integral_constant<int, 2>{});
+    else body(std::integral_constant<int, 4>{});
   }
 }
 

@@ -43,7 +43,7 @@ STK_API int stk_signed_step(const void* q, const void* k, const void* v, int dty
   STK_REQUIRE(why == nullptr, why ? why : "");
   uint64_t* keys = static_cast<uint64_t*>(workspace);
   const FrontArgs f = make_front_args(q, k, v, dtype, hq, hkv, n, b, d, lo, hi,
-                                      bounds_dtype != 0, predicted, sp, m, l, u, keys, s);
+                                      bounds_dtype != 0, predicted, sp, m, l, u, keys, s, false);
   STailArgs t{};
   t.kv = KV{q, k, v, hq, hkv, n, b, d};
   t.keys = keys; t.k = topk; t.ids = selected;

@@ -55,9 +55,11 @@ __device__ __forceinline__ void states_tok_wg(const StatesArgs& a, int wg,
                                               const Paging& pg = Paging{}) {
   using TT = TokTile<T, NCH, UP>;
   const int waves = blockDim.x / STK_WAVE;
-  const int64_t item = (int64_t)wg * waves + wave_id();
-  if (item >= (int64_t)a.hq * a.s) return;
-  const int h = (int)(item / a.s);
+  // (the states of 2^32 items would not fit the device: 32-bit divisions)
+  const uint32_t item32 = (uint32_t)wg * waves + __builtin_amdgcn_readfirstlane(wave_id());
+  if (item32 >= (uint64_t)a.hq * a.s) return;
+  const int64_t item = item32;
+  const int h = (int)(item32 / (uint32_t)a.s);
   TT t;
   t.init();
   uint32_t qw[TT::QW];
@@ -121,6 +123,96 @@ __device__ __forceinline__ void states_tok_wg(const StatesArgs& a, int wg,
       a.l[item] = l;
     }
     t.store(a.u + item * a.d, acc);
+  }
+}
+
+// Several slots of one query head per wave (B == CH), the tiles streamed
+// through one set of registers: the next block's K goes out as soon as this
+// block's logits are formed, its V as soon as this block's values are summed,
+// so the wave always has half a tile or more in flight.  The IDs and pages of
+// all IPW slots are fetched together, so a wave pays those two round trips
+// once instead of once per tile.
+// wg: workgroup index among those of KV row kv.
+template <typename T, int NCH, int UP, bool PG, int IPW>
+__device__ __forceinline__ void states_tok_multi(const StatesArgs& a, int kv, int wg,
+                                                 const Paging& pg = Paging{}) {
+  using TT = TokTile<T, NCH, UP>;
+  constexpr int D = TT::D;
+  const int per_head = (a.s + IPW - 1) / IPW, G = a.hq / a.hkv;
+  const int gi = wg * (int)(blockDim.x / STK_WAVE) + __builtin_amdgcn_readfirstlane(wave_id());
+  if (gi >= G * per_head) return;
+  const int hl = gi / per_head;
+  const int h = kv * G + hl, s0 = (gi - hl * per_head) * IPW;
+  const int cnt = a.s - s0 < IPW ? a.s - s0 : IPW;
+  const int64_t item0 = (int64_t)h * a.s + s0;
+  TT t;
+  t.init();
+  uint32_t qw[TT::QW];
+  // lane j holds slot s0 + j (lanes past the last slot repeat it)
+  const int j0 = lane_id() < cnt ? lane_id() : cnt - 1;
+  const int64_t bid = reinterpret_cast<const int32_t*>(a.ids)[item0 + j0];
+  t.load_q(reinterpret_cast<const T*>(a.q) + (size_t)h * D, qw);
+  const int nv = PG ? pg_blocks(pg, kv, a.n) : a.n;
+  const int rtok = PG ? pg_row_tokens(pg, kv) : 0;
+  const bool inrow = bid >= 0 && bid < a.n;
+  // page of this lane's block (dense: its row in K), -1 for the empty state,
+  // and the block's tokens holding data
+  int page, btok = a.b;
+  if constexpr (PG) {
+    btok = pg_block_tokens(rtok, bid, a.b);
+    page = pg_page(pg, kv, a.n, bid, inrow);
+    page = bid < nv && btok > 0 ? page : -1;
+  } else {
+    page = inrow ? (int)bid : -1;
+  }
+  const float scale = 1.0f / sqrtf((float)D);
+  const T* K = reinterpret_cast<const T*>(a.k);
+  const T* V = reinterpret_cast<const T*>(a.v);
+  auto tile = [&](int j) {
+    const int p = __builtin_amdgcn_readlane(page, j);
+    const size_t row = (PG ? 0 : (size_t)kv * a.n) + (size_t)(p < 0 ? 0 : p);
+    return row * TT::CH * D;
+  };
+  uint32_t kw[UP][TT::QW], vw[TT::CH][TT::VW];
+  size_t off = tile(0);
+  t.load_k(K + off, 0, kw);
+  t.load_v(V + off, 0, vw);
+#pragma unroll
+  for (int j = 0; j < IPW; ++j) {
+    const bool live = __builtin_amdgcn_readlane(page, j) >= 0;
+    const int lim = PG ? __builtin_amdgcn_readlane(btok, j) : TT::CH;
+    float s[UP], m = -INFINITY, l = 0.f, acc[TT::DPL];
+#pragma unroll
+    for (int e = 0; e < TT::DPL; ++e) acc[e] = 0.f;
+    t.scores(qw, kw, 0, lim, scale, s);
+    __builtin_amdgcn_sched_barrier(0);
+    if (j + 1 < IPW) {
+      off = tile(j + 1);
+      t.load_k(K + off, 0, kw);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (PG && lim < TT::CH)
+      t.template accumulate<false, false, true>(s, vw, m, l, acc, nullptr, lim);
+    else
+      t.template accumulate<false, false>(s, vw, m, l, acc);
+    __builtin_amdgcn_sched_barrier(0);
+    if (j + 1 < IPW) {
+      t.load_v(V + off, 0, vw);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (j < cnt) {
+      if (!live) {
+        m = -INFINITY;
+        l = 0.f;
+#pragma unroll
+        for (int e = 0; e < TT::DPL; ++e) acc[e] = 0.f;
+      }
+      if (lane_id() == 0) {
+        a.m[item0 + j] = m;
+        a.l[item0 + j] = l;
+      }
+      t.store(a.u + (item0 + j) * D, acc);
+    }
   }
 }
 

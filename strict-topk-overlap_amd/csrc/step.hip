@@ -55,7 +55,7 @@ const char* plan_step(int dtype, int hq, int hkv, int n, int b, int d, int topk,
 FrontArgs make_front_args(const void* q, const void* k, const void* v, int dtype, int hq,
                           int hkv, int n, int b, int d, const void* lo, const void* hi, int lb,
                           const void* predicted, int sp, float* m, float* l, float* u,
-                          uint64_t* keys, const StepShape& s) {
+                          uint64_t* keys, const StepShape& s, bool paged) {
   FrontArgs f{};
   f.sc.q = q; f.sc.qtype = dtype; f.sc.lo = lo; f.sc.hi = hi; f.sc.lb = lb;
   f.sc.hq = hq; f.sc.hkv = hkv; f.sc.n = n; f.sc.d = d;
@@ -64,8 +64,34 @@ FrontArgs make_front_args(const void* q, const void* k, const void* v, int dtype
   f.st.q = q; f.st.k = k; f.st.v = v; f.st.ids = predicted; f.st.itype = IT_I32;
   f.st.hq = hq; f.st.hkv = hkv; f.st.n = n; f.st.b = b; f.st.d = d; f.st.s = sp;
   f.st.m = m; f.st.l = l; f.st.u = u;
-  f.score_wgs = hkv * f.sc.chunks;
-  f.total_wgs = f.score_wgs + (int)(((int64_t)hq * sp + 3) / 4);
+  const int64_t chunks = (int64_t)hkv * f.sc.chunks, items = (int64_t)hq * sp;
+  const int G = hq / hkv;
+  // A grid that fills the GPU several times over is bound by throughput: its
+  // roles are laid out per KV row, a scoring workgroup takes several chunks
+  // with the next one's bounds in flight, and a paged states wave takes two
+  // slots (its table reads once for both; a third round trip that the dense
+  // wave does not have, where two slots were slower, 54.3 against 50.8 us at
+  // 64 heads x 96 slots x 8000 blocks).  Measured per step, single against
+  // multi: 24 ragged paged requests x 32 heads x 64 slots 174 -> 134 us;
+  // 2 requests x 512 blocks 20.8 -> 19.6; 8 KV heads alone (1024-4096 slots,
+  // at most 1024 chunks) 14.9 -> 15.4 and 25.1 -> 25.4, so those stay single.
+  f.multi = s.one && G <= kFrontMultiG &&
+            (items >= (paged && G > 1 ? 4096 : (paged ? 8192 : 2048)) || chunks >= 2048);
+  if (f.multi) {
+    // two slots per wave: 4096 slots 25.4 -> 26.1 us, 16384 slots 52.7 -> 50.8
+    f.ipw = paged && items >= 8192 ? 2 : 1;
+    // 4096 chunks: 1, 2, 4 per workgroup 104.9, 100.1, 103.6 us; 11656 (a ragged
+    // batch, mostly past its rows' ends): 29.9, 24.4, 21.2
+    f.cpw = chunks >= 8192 ? 4 : (chunks >= 2048 ? 2 : 1);
+    f.score_wgs = (f.sc.chunks + f.cpw - 1) / f.cpw;
+    f.total_wgs = f.score_wgs + (G * ((sp + f.ipw - 1) / f.ipw) + 3) / 4;
+    f.dealt = hkv % 8 == 0 || hkv >= 64;
+    f.grid = (f.dealt ? (hkv + 7) / 8 * 8 : hkv) * f.total_wgs;
+  } else {
+    f.score_wgs = (int)chunks;
+    f.total_wgs = f.grid = (int)(chunks + (items + 3) / 4);
+  }
+  f.score_share = (((uint64_t)f.score_wgs << 32) + f.total_wgs - 1) / f.total_wgs;
   return f;
 }
 
@@ -192,7 +218,7 @@ static int step_call(const void* q, const void* k, const void* v, int dtype, int
   STK_REQUIRE(why == nullptr, why ? why : "");
   uint64_t* keys = static_cast<uint64_t*>(workspace);
   const FrontArgs f = make_front_args(q, k, v, dtype, hq, hkv, n, b, d, lo, hi,
-                                      bounds_dtype != 0, predicted, sp, m, l, u, keys, s);
+                                      bounds_dtype != 0, predicted, sp, m, l, u, keys, s, false);
   TailArgs t{};
   t.kv = KV{q, k, v, hq, hkv, n, b, d};
   t.keys = keys; t.k = topk; t.ids = selected;

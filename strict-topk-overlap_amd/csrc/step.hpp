@@ -10,10 +10,18 @@
 
 namespace stk {
 
+constexpr int kFrontMultiG = 8;   // multi: query heads per KV head at most
+
 struct FrontArgs {
   ScoreArgs sc;
   StatesArgs st;
-  int score_wgs, total_wgs;
+  int grid;                    // workgroups
+  int score_wgs, total_wgs;    // of the launch; multi: of one KV row
+  uint64_t score_share;        // ceil(2^32 score_wgs / total_wgs)
+  bool multi;                  // a large grid (make_front_args)
+  int ipw;                     // multi: predicted slots per states wave
+  bool dealt;                  // multi: KV rows dealt over the XCDs
+  int cpw;                     // multi: chunks per scoring workgroup
   Paging pg;             // paged, batched KV (the PG kernels only)
 };
 
@@ -32,7 +40,7 @@ const char* plan_step(int dtype, int hq, int hkv, int n, int b, int d, int topk,
 FrontArgs make_front_args(const void* q, const void* k, const void* v, int dtype, int hq,
                           int hkv, int n, int b, int d, const void* lo, const void* hi, int lb,
                           const void* predicted, int sp, float* m, float* l, float* u,
-                          uint64_t* keys, const StepShape& s);
+                          uint64_t* keys, const StepShape& s, bool paged);
 
 // Launch k_front for (dtype, shape) on `st`.
 int launch_front(int dtype, const FrontArgs& f, const StepShape& s, hipStream_t st);

@@ -21,24 +21,55 @@
 
 namespace stk {
 
-template <typename T, int NCH, int UP, bool ONE, int P, int STEPS, int GT, bool PG>
+// MULTI: 0, or the predicted slots per states wave of a large grid.
+template <typename T, int NCH, int UP, bool ONE, int P, int STEPS, int GT, bool PG, int MULTI>
 __global__ __launch_bounds__(256, NCH <= 4 ? 4 : 2) void k_front(FrontArgs a) {
   // Workgroups are dealt round-robin over the 8 XCDs; roles are interleaved
   // on an XCD-contiguous logical index, so every XCD gets an even mix of
   // scoring and speculation work (and, with G query heads per KV head, the
   // scoring and the states of one KV head land on the same XCD's L2).
-  const int i = xcd_remap(blockIdx.x, gridDim.x);
-  // score workgroups among logical indices [0, i) and [0, i]
-  const int before = (int)(((int64_t)i * a.score_wgs) / a.total_wgs);
-  const int upto = (int)(((int64_t)(i + 1) * a.score_wgs) / a.total_wgs);
-  if (upto > before)
-    score_wg<T, P, STEPS, true, GT, PG>(a.sc, before, a.pg);
-  else
-    states_tok_wg<T, NCH, UP, int32_t, ONE, PG>(a.st, i - upto, a.pg);
+  //
+  // Score workgroups among logical indices [0, i): i times the share of score
+  // workgroups, a 32.32 fixed-point number rounded up, so that the count runs
+  // from 0 to score_wgs in steps of 0 and 1.
+  if constexpr (MULTI > 0) {
+    // the index runs over one KV row's workgroups; with `dealt`, the rows are
+    // dealt over the XCDs (a batch's long and short requests evenly), else
+    // each XCD has a contiguous range
+    int row, u;
+    if (a.dealt) {
+      const int p = (int)(blockIdx.x >> 3), r8 = p / a.total_wgs;
+      row = r8 * 8 + (int)(blockIdx.x & 7);
+      if (row >= a.sc.hkv) return;
+      // each row's roles start one later than the last row's: a period that
+      // divides the CUs of an XCD would give some CUs only one role (113 -> 141
+      // us at 24 requests whose rows alternate the roles over 32 workgroups)
+      u = (p - r8 * a.total_wgs + r8) % a.total_wgs;
+    } else {
+      const int i = xcd_remap(blockIdx.x, gridDim.x);
+      row = i / a.total_wgs;
+      u = i - row * a.total_wgs;
+    }
+    const int before = (int)(((uint64_t)u * a.score_share) >> 32);
+    const int upto = (int)(((uint64_t)(u + 1) * a.score_share) >> 32);
+    constexpr int GM = GT == 1 ? 1 : (P <= 2 && GT == 2 ? 2 : kFrontMultiG);
+    if (upto > before)
+      score_wg_multi<T, P, STEPS, GT, GM, PG>(a.sc, row, before * a.cpw, a.cpw, a.pg);
+    else
+      states_tok_multi<T, NCH, UP, PG, MULTI>(a.st, row, u - upto, a.pg);
+  } else {
+    const int i = xcd_remap(blockIdx.x, gridDim.x);
+    const int before = (int)(((uint64_t)i * a.score_share) >> 32);
+    const int upto = (int)(((uint64_t)(i + 1) * a.score_share) >> 32);
+    if (upto > before)
+      score_wg<T, P, STEPS, true, GT, PG>(a.sc, before, a.pg);
+    else
+      states_tok_wg<T, NCH, UP, int32_t, ONE, PG>(a.st, i - upto, a.pg);
+  }
 }
 
 template <typename T, int NCH, int UP, bool ONE, int KPT, int RPT, bool PG>
-__global__ __launch_bounds__(kTailThreads) void k_tail(TailArgs a) {
+__global__ __launch_bounds__(kTailThreads, KPT == 4 && RPT == 4 && NCH <= 4 ? 4 : 1) void k_tail(TailArgs a) {
   tail_head<T, NCH, UP, ONE, KPT, RPT, PG>(a);
 }
 
@@ -49,16 +80,27 @@ __global__ __launch_bounds__(kTailThreads) void k_stail(STailArgs a) {
 
 namespace launch {
 
+template <bool PG, typename T, int NCH, int UP, bool ONE, int P, int STEPS, int MULTI>
+int front_multi(const FrontArgs& f, const StepShape& s, hipStream_t st) {
+  const dim3 grid(f.grid), block(256);
+  if (s.gt == 1)
+    hipLaunchKernelGGL((k_front<T, NCH, UP, ONE, P, STEPS, 1, PG, MULTI>), grid, block, 0, st, f);
+  else if (s.gt == 2)
+    hipLaunchKernelGGL((k_front<T, NCH, UP, ONE, P, STEPS, 2, PG, MULTI>), grid, block, 0, st, f);
+  else
+    hipLaunchKernelGGL((k_front<T, NCH, UP, ONE, P, STEPS, 4, PG, MULTI>), grid, block, 0, st, f);
+  return stk_check_launch("k_front");
+}
+
 template <bool PG, typename T, int NCH, int UP, bool ONE, int P, int STEPS>
 int front_gt(const FrontArgs& f, const StepShape& s, hipStream_t st) {
-  const dim3 grid(f.total_wgs), block(256);
-  if (s.gt == 1)
-    hipLaunchKernelGGL((k_front<T, NCH, UP, ONE, P, STEPS, 1, PG>), grid, block, 0, st, f);
-  else if (s.gt == 2)
-    hipLaunchKernelGGL((k_front<T, NCH, UP, ONE, P, STEPS, 2, PG>), grid, block, 0, st, f);
-  else
-    hipLaunchKernelGGL((k_front<T, NCH, UP, ONE, P, STEPS, 4, PG>), grid, block, 0, st, f);
-  return stk_check_launch("k_front");
+  if constexpr (ONE)
+    if (f.multi) {
+      if constexpr (PG)
+        if (f.ipw == 2) return front_multi<PG, T, NCH, UP, ONE, P, STEPS, 2>(f, s, st);
+      return front_multi<PG, T, NCH, UP, ONE, P, STEPS, 1>(f, s, st);
+    }
+  return front_multi<PG, T, NCH, UP, ONE, P, STEPS, 0>(f, s, st);
 }
 
 template <bool PG, typename T, int NCH>
@@ -74,7 +116,7 @@ int front_t(const FrontArgs& f, const StepShape& s, hipStream_t st) {
 
 template <bool PG>
 int front(int dtype, const FrontArgs& f, const StepShape& s, hipStream_t st) {
-  if (f.total_wgs == 0) return STK_OK;
+  if (f.grid == 0) return STK_OK;
   STK_DISPATCH_STEP(dtype, s.nch, { return front_t<PG, T, NCH>(f, s, st); });
   return STK_EINVAL;
 }

@@ -83,6 +83,10 @@ struct TokTile {
   // offset from one base per lane and no address needs a clamp.
   __device__ __forceinline__ void load(const T* kb, const T* vb, int t0,
                                        uint32_t (&kw)[UP][QW], uint32_t (&vw)[CH][VW]) const {
+    load_k(kb, t0, kw);
+    load_v(vb, t0, vw);
+  }
+  __device__ __forceinline__ void load_k(const T* kb, int t0, uint32_t (&kw)[UP][QW]) const {
     const T* krow = kb + (size_t)(t0 + slot) * D;
 #pragma unroll
     for (int u = 0; u < UP; ++u) {
@@ -93,6 +97,8 @@ struct TokTile {
         kw[u][4 * c + 3] = x.w;
       }
     }
+  }
+  __device__ __forceinline__ void load_v(const T* vb, int t0, uint32_t (&vw)[CH][VW]) const {
     const T* vrow = vb + (size_t)t0 * D + lane_id() * DPL;
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
@@ -133,7 +139,14 @@ struct TokTile {
       for (int w = 0; w < QW; ++w) acc = Elem<T>::dot(kw[u][w], qw[w], acc);
       acc = quad_sum(acc);
       int t = t0 + slot + TPP * u;
-      s[u] = t < B ? acc * scale : -INFINITY;
+      {
+        // a logit of its own: fused into the exponent's subtraction in one
+        // kernel and not in another, the same block's states would differ
+        // in their last bits
+#pragma clang fp contract(off)
+        acc = acc * scale;
+      }
+      s[u] = t < B ? acc : -INFINITY;
     }
   }
 
