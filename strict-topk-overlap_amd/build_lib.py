@@ -2,9 +2,9 @@
 
 Usage: python strict-topk-overlap_amd/build_lib.py [--jobs N]
 
-Objects go to strict-topk-overlap_amd/_build/, the shared library next to the
-Python package (strict_topk/libstrict_topk_hip.so), so it travels with the
-source tree.
+Objects go to strict-topk-overlap_amd/_build/, the shared library and the native
+host module next to the Python package (strict_topk/libstrict_topk_hip.so,
+strict_topk/_host.so), so they travel with the source tree.
 """
 from __future__ import annotations
 
@@ -14,11 +14,13 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 ROOT = Path(__file__).resolve().parent
 CSRC = ROOT / "csrc"
 OUT = ROOT / "strict_topk" / "libstrict_topk_hip.so"
+HOST = ROOT / "strict_topk" / "_host.so"
 BUILD = ROOT / "_build"
 ARCH = "gfx950"
 SOURCES = ["api.cpp", "states.hip", "select.hip", "repair.hip", "signed.hip", "hier.hip", "sstep.hip",
@@ -66,11 +68,34 @@ def _compile(src: str) -> Path:
     return obj
 
 
+def build_host() -> Path:
+    """The native host path (csrc/host.cpp), a Python extension module over
+    torch's C++ tensors; no device code."""
+    import torch
+    root = Path(torch.__file__).resolve().parent
+    tmp = HOST.with_suffix(".so.tmp")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
+           "-Wno-sign-compare", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-isystem{root / 'include'}",
+           f"-isystem{root / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",
+           "-isystem/opt/rocm/include", f"-isystem{sysconfig.get_path('include')}",
+           str(CSRC / "host.cpp"), "-o", str(tmp), f"-L{root / 'lib'}", "-ltorch_python",
+           "-ltorch_cpu", "-ltorch", "-lc10", "-lc10_hip"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"host module failed:\n{res.stderr}")
+    os.replace(tmp, HOST)
+    return HOST
+
+
 def build(jobs: int | None = None) -> Path:
     BUILD.mkdir(exist_ok=True)
     jobs = jobs or min(len(SOURCES), os.cpu_count() or 4)
     with cf.ThreadPoolExecutor(max_workers=jobs) as ex:
+        host = ex.submit(build_host)
         objs = list(ex.map(_compile, SOURCES))
+        host.result()
     tmp = OUT.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp),
            *map(str, objs)]

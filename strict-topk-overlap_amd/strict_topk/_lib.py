@@ -114,6 +114,27 @@ def lib():
     return _lib
 
 
+_host = None
+
+
+def host():
+    """The native host path of the fused steps (csrc/host.cpp): its functions
+    return None for calls that the Python code has to check or refuse."""
+    global _host
+    if _host is None:
+        handle = lib()
+        try:
+            from . import _host as module
+        except ImportError as e:
+            raise RuntimeError("strict_topk native host module not built (run `python "
+                               "strict-topk-overlap_amd/build_lib.py`)") from e
+        module.bind(*(ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in (
+            "stk_step_supported", "stk_step_workspace_bytes", "stk_speculative_step",
+            "stk_paged_workspace_bytes", "stk_paged_step", "stk_paged_signed_step")))
+        _host = module
+    return _host
+
+
 def ptr(t):
     """Device address of a tensor, or None."""
     return None if t is None else t.data_ptr()
@@ -149,14 +170,19 @@ def workspace(nbytes, device):
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
 
 
+def fail(rc):
+    """Raise the exception of a C entry point's status."""
+    msg = lib().stk_last_error().decode(errors="replace")
+    if rc == -1:
+        raise ValueError(msg)
+    raise RuntimeError(msg)
+
+
 def call(name, *args):
     fn = getattr(lib(), name)
     rc = fn(*args)
     if rc != 0:
-        msg = lib().stk_last_error().decode(errors="replace")
-        if rc == -1:
-            raise ValueError(msg)
-        raise RuntimeError(msg)
+        fail(rc)
     return rc
 
 
@@ -178,3 +204,4 @@ def prepare(device):
     with torch.cuda.device(idx):
         call("stk_step_prepare")
     _prepared.add(idx)
+    host().prepared(idx)

@@ -229,10 +229,28 @@ def _common(q, kv, predicted, topk):
     return head, selected, state, st, out, ws
 
 
+def _native(q, kv, predicted, topk, mode, tau=0.0, min_remaining=0.0, tol=0.0, eps=0.0):
+    """The call on the native host path, or None where the code below has to
+    check or refuse it."""
+    if type(kv) is not PagedKV:
+        return None
+    got = _lib.host().paged_step(q, kv.k_pages, kv.v_pages, kv.lo_pages, kv.hi_pages,
+                                 kv.block_table, kv.nblocks, kv.ntokens, predicted, topk, mode,
+                                 tau, min_remaining, tol, eps)
+    if type(got) is int:
+        _lib.fail(got)
+    return got
+
+
 def speculative_step(q, kv, predicted, topk, union=False):
     """The batched ``step.speculative_step``: per request, select(q, lo, hi,
     topk) || partials(q, k, v, predicted), then the saved (or union) repair.
     q [R, Hq, D], predicted [R, Hq, SP] int32 logical IDs; results [R, Hq, ...]."""
+    if predicted is not None:
+        got = _native(q, kv, predicted, topk, 1 if union else 0)
+        if got is not None:
+            sel, m, l, u, out = got
+            return StepResult(sel, PartialState(m, l, u), out)
     head, selected, state, st, out, ws = _common(q, kv, predicted, topk)
     _lib.call("stk_paged_step", *head, 1 if union else 0, _lib.ptr(selected), *st,
               _lib.ptr(out), _lib.ptr(ws), ws.numel(), _lib.stream(q.device))
@@ -243,6 +261,9 @@ def exact(q, kv, topk):
     """The serial path over the batch: the top-K of the bound scores, then the
     exact attention over the selected blocks (no prediction).  Returns
     (selected [R, Hq, topk], out [R, Hq, D])."""
+    got = _native(q, kv, None, topk, 0)
+    if got is not None:
+        return got[0], got[4]
     head, selected, _, st, out, ws = _common(q, kv, None, topk)
     _lib.call("stk_paged_step", *head, 0, _lib.ptr(selected), *st, _lib.ptr(out),
               _lib.ptr(ws), ws.numel(), _lib.stream(q.device))
@@ -259,6 +280,13 @@ def speculative_signed_step(q, kv, predicted, topk, mode="hybrid", mass_threshol
         raise ValueError("mass_threshold must be in [0,1]")
     if not 0 <= max_extra_mass <= 1:
         raise ValueError("max_extra_mass must be in [0,1]")
+    if predicted is not None:
+        got = _native(q, kv, predicted, topk, 3 if mode == "hybrid" else 2, mass_threshold,
+                      min_remaining, cancellation_tol, max_extra_mass)
+        if got is not None:
+            sel, m, l, u, out, bad, rem, approx, extra, pos, tot = got
+            return SignedStepResult(sel, PartialState(m, l, u),
+                                    SignedRepairResult(out, bad, rem, approx, extra, pos, tot))
     head, selected, state, st, out, ws = _common(q, kv, predicted, topk)
     r, hq = q.shape[:2]
     dev = q.device

@@ -93,6 +93,12 @@ def speculative_step(q, k, v, lo, hi, predicted, topk, union=False):
     Validation follows ``gqa.select_blocks`` and ``gqa.partials`` (same
     ValueError messages).  ``union`` selects ``repair_union`` semantics.
     """
+    got = _lib.host().speculative_step(q, k, v, lo, hi, predicted, topk, union)
+    if got is not None:
+        if type(got) is int:
+            _lib.fail(got)
+        sel, m, l, u, out = got
+        return StepResult(sel, PartialState(m, l, u), out)
     gqa._shape(q, k, v, predicted)
     _check_bounds(q, k, lo, hi)
     topk = int(topk)
