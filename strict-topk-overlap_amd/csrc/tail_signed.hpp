@@ -74,6 +74,10 @@ __device__ __forceinline__ void stail_head(const STailArgs& a) {
   constexpr int SW = kTailMaxK / STK_WAVE;   // slot words of wave 0
   // two tile buffers in flight when they fit the register budget
   constexpr bool DB = ONE && RPT == 4 && UP * TT::QW + 4 * TT::NV <= 64;
+  // the u rows are held from entry where the registers allow it; sixteen of
+  // them beside a D = 256 tile do not fit (with B = 16 the spilling build
+  // gave wrong sums for rows past SP): those are read where they are summed
+  constexpr bool LATE = NCH == 8 && RPT == 16;
   __shared__ int map[kTailMapN];
   __shared__ int sel[kTailMaxK], miss[kTailMaxK], pids[kTailMaxK];
   __shared__ float s_pm[kTailMaxK], s_pl[kTailMaxK];
@@ -122,12 +126,15 @@ __device__ __forceinline__ void stail_head(const STailArgs& a) {
   const float pmv = ld_or(a.pm, (int64_t)h * sp + tid, tid < sp, -INFINITY);
   const float plv = ld_or(a.pl, (int64_t)h * sp + tid, tid < sp, 0.f);
   const int c4 = tid % TPR, rg = tid / TPR;
-  float4 uu[RPT];
-#pragma unroll
-  for (int j = 0; j < RPT; ++j) {
+  auto u_row = [&](int j) {
     const int r = rg + RG * j;
     const int64_t row = (int64_t)h * sp + (r < sp ? r : 0);
-    uu[j] = *reinterpret_cast<const float4*>(a.pu + row * D + 4 * c4);
+    return *reinterpret_cast<const float4*>(a.pu + row * D + 4 * c4);
+  };
+  float4 uu[LATE ? 1 : RPT];
+  if constexpr (!LATE) {
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) uu[j] = u_row(j);
   }
   // ---- membership map (max predicted slot + 1 per block ID), cleared here
   // and filled between the top-K's first two barriers
@@ -344,7 +351,7 @@ __device__ __forceinline__ void stail_head(const STailArgs& a) {
   float hl = 0.f, nl = 0.f, sl = 0.f;
   float4 hu = make_float4(0.f, 0.f, 0.f, 0.f);
   float4 lu = hu, la = hu, nu = hu, su = hu;
-#pragma unroll
+#pragma unroll (LATE ? 4 : RPT)
   for (int j = 0; j < RPT; ++j) {
     const int r = rg + RG * j;   // < 16 * RG <= 512
     const int rr = r < kTailMaxK ? r : 0;
@@ -364,7 +371,8 @@ __device__ __forceinline__ void stail_head(const STailArgs& a) {
     const float wn = wr ? wl : 0.f;
     const float ws = us ? wexp(pm, mu) : 0.f;
     // rows past sp were loaded from row 0 (or a stand-in buffer): zero them
-    const float4 u4 = r < sp ? uu[j] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 ux = LATE ? u_row(j) : uu[LATE ? 0 : j];
+    const float4 u4 = r < sp ? ux : make_float4(0.f, 0.f, 0.f, 0.f);
     hl += wk * pl;
     nl += wn * pl;
     sl += ws * pl;

@@ -65,6 +65,7 @@ def _alone(kv, r):
     (5, 8, 8, 32, 128, 2200, 4, 64, BF, "keys"),      # many chunks, two per workgroup
     (33, 8, 8, 16, 256, 500, 2, 8, BF, "fp32"),       # four chunks per workgroup, D = 256
     (9, 64, 8, 16, 128, 90, 31, 20, BF, "keys"),      # eight heads per KV head
+    (3, 2, 1, 16, 64, 4500, 40, 50, BF, "keys"),      # rows of more than 4096 keys
 ])
 def test_batch_equals_single_requests(requests, hq, hkv, b, d, longest, sp, topk, dtype, bounds):
     from strict_topk import paged
@@ -107,4 +108,42 @@ def test_dense_front_equals_the_separate_calls(hq, hkv, n, b, d, sp, topk, dtype
     assert torch.equal(got.selected, ids)
     for x, y in ((got.state.m, st.m), (got.state.l, st.l), (got.state.u, st.u),
                  (got.output, gqa.exact(q, k, v, ids))):
+        torch.testing.assert_close(x, y, rtol=3e-4, atol=3e-4)
+
+
+@pytest.mark.parametrize("d,sp,n", [
+    (128, 64, 300), (128, 65, 300), (128, 128, 300), (128, 129, 300),   # 4, 8, 8, 16 row passes
+    (256, 33, 200), (256, 64, 200), (256, 65, 200), (64, 129, 400), (64, 256, 400),
+    (128, 40, 4096), (128, 40, 4097), (128, 129, 4097), (64, 200, 8192),  # 512 / 1024 threads
+])
+def test_tails_at_row_and_key_edges(d, sp, n):
+    """The two-launch tails at the edges of their predicted-row passes and of
+    their thread counts, against the separate calls (five query heads per KV
+    head, so the one-launch step does not take the shape)."""
+    from strict_topk import gqa, gqa_light, kernels, signed_fused, step
+    hq, hkv, b, topk = 10, 2, 16, 37
+    gen = torch.Generator(device=DEV).manual_seed(d + sp + n)
+    q = torch.randn((hq, d), generator=gen, device=DEV, dtype=BF)
+    k = torch.randn((hkv, n, b, d), generator=gen, device=DEV, dtype=BF)
+    v = torch.randn((hkv, n, b, d), generator=gen, device=DEV, dtype=BF)
+    lo, hi = k.amin(2), k.amax(2)
+    ids = gqa.select_blocks(q, lo.float(), hi.float(), topk)
+    noise = torch.rand((hq, n), generator=gen, device=DEV)
+    noise.scatter_(1, ids[:, : topk * 2 // 3].long(), 2.0)      # two thirds predicted
+    p = noise.topk(sp, dim=1).indices.to(torch.int32).contiguous()
+    got = step.speculative_step(q, k, v, lo, hi, p, topk)
+    st = gqa.partials(q, k, v, p)
+    assert torch.equal(got.selected, ids)
+    for x, y in ((got.state.u, st.u),
+                 (got.output, gqa_light.repair_saved_light(q, k, v, ids, p, st)),
+                 (got.output, gqa.exact(q, k, v, ids))):
+        torch.testing.assert_close(x, y, rtol=3e-4, atol=3e-4)
+    sg = step.speculative_signed_step(q, k, v, lo, hi, p, topk, "hybrid", 0.02)
+    pred = kernels.speculate(q, k, v, p, "hybrid", 0.02, keep_mass=True)
+    want = signed_fused.repair_signed_fused(q, k, v, ids, p, pred)
+    assert torch.equal(sg.selected, ids)
+    assert torch.equal(sg.result.positive_jobs, want.positive_jobs)
+    assert torch.equal(sg.result.total_jobs, want.total_jobs)
+    for x, y in ((sg.result.output, want.output), (sg.result.output, gqa.exact(q, k, v, ids)),
+                 (sg.result.remaining, want.remaining)):
         torch.testing.assert_close(x, y, rtol=3e-4, atol=3e-4)
