@@ -18,6 +18,7 @@ template <typename T, int NCH, int UP>
 void launch_t(const GqaRepairArgs& g, int rpt, hipStream_t st) {
   const dim3 grid(g.kv.hq), block(kTailThreads);
   if (rpt == 4) hipLaunchKernelGGL((k_repair_fast<T, NCH, UP, 4>), grid, block, 0, st, g);
+  else if (rpt == 8) hipLaunchKernelGGL((k_repair_fast<T, NCH, UP, 8>), grid, block, 0, st, g);
   else hipLaunchKernelGGL((k_repair_fast<T, NCH, UP, 16>), grid, block, 0, st, g);
 }
 

@@ -28,7 +28,7 @@ namespace stk {
 inline int repair_fast_rpt(int sp, int d) {
   const int per_pass = kTailThreads * 4 / d;
   const int rows = (sp + per_pass - 1) / per_pass;
-  return rows <= 4 ? 4 : (rows <= 16 ? 16 : 0);
+  return rows <= 4 ? 4 : (rows <= 8 ? 8 : (rows <= 16 ? 16 : 0));
 }
 
 template <typename T, int NCH, int UP, int RPT>

@@ -528,6 +528,8 @@ int srepair_one(const SRepairArgs& a, int rpt, hipStream_t st) {
   const dim3 grid(a.kv.hq), block(kTailThreads);
   if (rpt == 4)
     hipLaunchKernelGGL((k_srepair<T, NCH, UP, ONE, 4, COMPACT>), grid, block, 0, st, a);
+  else if (rpt == 8)
+    hipLaunchKernelGGL((k_srepair<T, NCH, UP, ONE, 8, COMPACT>), grid, block, 0, st, a);
   else
     hipLaunchKernelGGL((k_srepair<T, NCH, UP, ONE, 16, COMPACT>), grid, block, 0, st, a);
   return stk_check_launch("k_srepair");
@@ -540,7 +542,8 @@ int srepair_launch(int dtype, const SRepairArgs& a, hipStream_t st) {
   const int up = tok_up(b);
   const bool one = b == 16 * up;
   const int per_pass = kTailThreads * 4 / d;
-  const int rpt = (rows + per_pass - 1) / per_pass <= 4 ? 4 : 16;
+  const int passes = (rows + per_pass - 1) / per_pass;
+  const int rpt = passes <= 4 ? 4 : (passes <= 8 ? 8 : 16);
   STK_DISPATCH_STEP(dtype, nch, {
     return up == 1 ? (one ? srepair_one<T, NCH, 1, true, COMPACT>(a, rpt, st)
                           : srepair_one<T, NCH, 1, false, COMPACT>(a, rpt, st))

@@ -29,6 +29,7 @@ struct FrontArgs {
 struct StepShape {
   int nch, passes, steps, gt, kpt, up, rpt;
   bool one;
+  bool wide;   // k_tail with 1024 threads (its rpt: 4)
 };
 
 // Shape plan of a fused step, or a message saying why it is not supported.

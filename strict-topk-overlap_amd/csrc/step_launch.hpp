@@ -68,9 +68,10 @@ __global__ __launch_bounds__(256, NCH <= 4 ? 4 : 2) void k_front(FrontArgs a) {
   }
 }
 
-template <typename T, int NCH, int UP, bool ONE, int KPT, int RPT, bool PG>
-__global__ __launch_bounds__(kTailThreads, KPT == 4 && RPT == 4 && NCH <= 4 ? 4 : 1) void k_tail(TailArgs a) {
-  tail_head<T, NCH, UP, ONE, KPT, RPT, PG>(a);
+template <typename T, int NCH, int UP, bool ONE, int KPT, int RPT, bool PG, int TH>
+__global__ __launch_bounds__(TH, (KPT == 4 && RPT == 4 && NCH <= 4) || TH > 512 ? 4 : 1)
+void k_tail(TailArgs a) {
+  tail_head<T, NCH, UP, ONE, KPT, RPT, PG, TH>(a);
 }
 
 template <typename T, int NCH, int UP, bool ONE, int KPT, int RPT, bool PG>
@@ -123,16 +124,24 @@ int front(int dtype, const FrontArgs& f, const StepShape& s, hipStream_t st) {
 
 template <bool PG, typename T, int NCH, int UP, bool ONE>
 int tail_one(const TailArgs& t, const StepShape& s, hipStream_t st) {
-  const dim3 grid(t.kv.hq), block(kTailThreads);
-#define STK_TAIL(KPT)                                                                   \
-  if (s.rpt == 4)                                                                       \
-    hipLaunchKernelGGL((k_tail<T, NCH, UP, ONE, KPT, 4, PG>), grid, block, 0, st, t);   \
-  else                                                                                  \
-    hipLaunchKernelGGL((k_tail<T, NCH, UP, ONE, KPT, 16, PG>), grid, block, 0, st, t);
+  const dim3 grid(t.kv.hq), block(s.wide ? 2 * kTailThreads : kTailThreads);
+#define STK_TAIL_AT(KPT, RPT, TH) \
+  hipLaunchKernelGGL((k_tail<T, NCH, UP, ONE, KPT, RPT, PG, TH>), grid, block, 0, st, t)
+#define STK_TAIL(KPT)                                             \
+  if (s.rpt == 4) STK_TAIL_AT(KPT, 4, kTailThreads);              \
+  else if (s.rpt == 8) STK_TAIL_AT(KPT, 8, kTailThreads);         \
+  else STK_TAIL_AT(KPT, 16, kTailThreads);
+  if constexpr (NCH <= 4) {
+    if (s.wide) {
+      STK_TAIL_AT(8, 4, 2 * kTailThreads);
+      return stk_check_launch("k_tail");
+    }
+  }
   if (s.kpt == 4) { STK_TAIL(4) }
   else if (s.kpt == 8) { STK_TAIL(8) }
   else { STK_TAIL(16) }
 #undef STK_TAIL
+#undef STK_TAIL_AT
   return stk_check_launch("k_tail");
 }
 
@@ -153,6 +162,8 @@ int stail_one(const STailArgs& t, const StepShape& s, hipStream_t st) {
 #define STK_STAIL(KPT)                                                                  \
   if (s.rpt == 4)                                                                       \
     hipLaunchKernelGGL((k_stail<T, NCH, UP, ONE, KPT, 4, PG>), grid, block, 0, st, t);  \
+  else if (s.rpt == 8)                                                                  \
+    hipLaunchKernelGGL((k_stail<T, NCH, UP, ONE, KPT, 8, PG>), grid, block, 0, st, t);  \
   else                                                                                  \
     hipLaunchKernelGGL((k_stail<T, NCH, UP, ONE, KPT, 16, PG>), grid, block, 0, st, t);
   if (s.kpt == 4) { STK_STAIL(4) }

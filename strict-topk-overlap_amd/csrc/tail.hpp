@@ -53,21 +53,23 @@ struct TailArgs {
 // selected (the rest of the ID row is -1).  The pages of the row's blocks are
 // loaded with the keys, so a selected block's page is known the moment the
 // top-K names it, with no extra round trip before its tile.
-template <typename T, int NCH, int UP, bool ONE, int KPT, int RPT, bool PG = false>
+template <typename T, int NCH, int UP, bool ONE, int KPT, int RPT, bool PG = false,
+          int TH = kTailThreads>
 __device__ __forceinline__ void tail_head(const TailArgs& a) {
   using TT = TokTile<T, NCH, UP>;
+  constexpr int TW = TH / STK_WAVE;
   constexpr int D = TT::D;
   constexpr int TPR = D / 4;              // threads per state row (16-byte loads)
-  constexpr int RG = kTailThreads / TPR;  // rows per pass of the state prefetch
+  constexpr int RG = TH / TPR;  // rows per pass of the state prefetch
   __shared__ int map[kTailMapN];
   __shared__ int sel[kTailMaxK], miss[kTailMaxK], pids[kTailMaxK];
   __shared__ float s_pm[kTailMaxK], s_pl[kTailMaxK];
   __shared__ TopkBinsLds tb;
-  __shared__ int s_scan[kTailWaves];
+  __shared__ int s_scan[TW];
   // the hits' partial sums, one row per wave (relative to the wave's max)
-  __shared__ float s_hmax[kTailWaves], s_hl[kTailWaves];
-  __shared__ __align__(16) float s_hu[kTailWaves][D];
-  __shared__ float s_wm[kTailWaves], s_wl[kTailWaves], s_wu[kTailWaves][D];
+  __shared__ float s_hmax[TW], s_hl[TW];
+  __shared__ __align__(16) float s_hu[TW][D];
+  __shared__ float s_wm[TW], s_wl[TW], s_wu[TW][D];
   __shared__ int mtk[PG ? kTailMaxK : 1];   // PG: tokens of each listed miss
   const int h = xcd_remap(blockIdx.x, gridDim.x);   // a KV group's heads on one XCD
   const int nrow = a.kv.n, sp = a.sp;
@@ -108,7 +110,7 @@ __device__ __forceinline__ void tail_head(const TailArgs& a) {
   }
   // ---- membership map (max predicted slot + 1 per block ID), cleared here
   // and filled between the top-K's first two barriers
-  for (int i = tid; i < n; i += kTailThreads) map[i] = 0;
+  for (int i = tid; i < n; i += TH) map[i] = 0;
   // every slot entry is written (empty past sp): the row sums below read
   // entries past sp with zero weight, and LDS holds whatever an earlier
   // workgroup left there (NaN patterns included, and 0 * NaN is NaN)
@@ -188,7 +190,7 @@ __device__ __forceinline__ void tail_head(const TailArgs& a) {
   if (ONE && w < nm) t.load(K + tile(w), V + tile(w), 0, kw, vw);
   // the selected IDs go out behind the tile loads (stores count in the same
   // vector memory counter, so stores issued before the drain would hold it)
-  for (int i = tid; i < a.k; i += kTailThreads)
+  for (int i = tid; i < a.k; i += TH)
     a.ids[(size_t)h * a.k + i] = (!PG || i < kk) ? sel[i] : -1;
   // ---- the hits' (or, for union, every predicted row's) partial LSE sums:
   // saved mode takes slot p when P[p] is selected and p is the highest slot
@@ -247,7 +249,7 @@ __device__ __forceinline__ void tail_head(const TailArgs& a) {
   float m = -INFINITY, l = 0.f, acc[TT::DPL];
 #pragma unroll
   for (int e = 0; e < TT::DPL; ++e) acc[e] = 0.f;
-  for (int x = w; x < nm; x += kTailWaves) {
+  for (int x = w; x < nm; x += TW) {
     // PG: a partly filled block weights only its first mtk[x] tokens
     const int lim = PG ? mtk[x] : a.kv.b;
     if constexpr (ONE) {
@@ -272,10 +274,10 @@ __device__ __forceinline__ void tail_head(const TailArgs& a) {
   if (tid < D) {
     float M = -INFINITY;
 #pragma unroll
-    for (int x = 0; x < kTailWaves; ++x) M = fmaxf(M, fmaxf(s_hmax[x], s_wm[x]));
+    for (int x = 0; x < TW; ++x) M = fmaxf(M, fmaxf(s_hmax[x], s_wm[x]));
     float num = 0.f, den = 0.f;
 #pragma unroll
-    for (int x = 0; x < kTailWaves; ++x) {
+    for (int x = 0; x < TW; ++x) {
       const float fh = wexp(s_hmax[x], M), f = wexp(s_wm[x], M);
       num += fh * s_hu[x][tid] + f * s_wu[x][tid];
       den += fh * s_hl[x] + f * s_wl[x];
