@@ -77,14 +77,18 @@ FrontArgs make_front_args(const void* q, const void* k, const void* v, int dtype
   // slots (its table reads once for both; a third round trip that the dense
   // wave does not have, where two slots were slower, 54.3 against 50.8 us at
   // 64 heads x 96 slots x 8000 blocks).  Measured per step, single against
-  // multi: 24 ragged paged requests x 32 heads x 64 slots 174 -> 134 us;
-  // 2 requests x 512 blocks 20.8 -> 19.6; 8 KV heads alone (1024-4096 slots,
-  // at most 1024 chunks) 14.9 -> 15.4 and 25.1 -> 25.4, so those stay single.
-  f.multi = s.one && G <= kFrontMultiG &&
-            (items >= (paged && G > 1 ? 4096 : (paged ? 8192 : 2048)) || chunks >= 2048);
+  // multi: 24 ragged paged requests x 32 heads x 64 slots 174 -> 134 us; 8
+  // requests x 64 heads x 64 slots 63.2 -> 58.1.  With up to four query heads
+  // per KV head the middle sizes lose (32 heads, 8-16 requests of 200-500
+  // blocks, 10752-16384 slots, D = 128: 33.0 -> 33.5, 41.0 -> 42.0), so those
+  // stay single up to 24576 slots (12 requests x 32 heads x 53 slots, D = 256:
+  // 146 -> 121); dense grids gain 2 % from 2048 slots.
+  const int64_t least = !paged ? 2048 : (G > 4 || d > 128 ? 4096 : 24576);
+  f.multi = s.one && G <= kFrontMultiG && (items >= least || chunks >= 2048);
   if (f.multi) {
-    // two slots per wave: 4096 slots 25.4 -> 26.1 us, 16384 slots 52.7 -> 50.8
-    f.ipw = paged && items >= 8192 ? 2 : 1;
+    // two slots per wave: 4096 slots 25.4 -> 26.1 us, 16384 slots 52.7 -> 50.8;
+    // 8192 slots beside 2048 chunks 41.6 -> 38.7
+    f.ipw = paged && items >= 8192 && (items >= 16384 || chunks >= 2048) ? 2 : 1;
     // 4096 chunks: 1, 2, 4 per workgroup 104.9, 100.1, 103.6 us; 11656 (a ragged
     // batch, mostly past its rows' ends): 29.9, 24.4, 21.2
     f.cpw = chunks >= 8192 ? 4 : (chunks >= 2048 ? 2 : 1);

@@ -351,7 +351,7 @@ __device__ __forceinline__ void stail_head(const STailArgs& a) {
   float hl = 0.f, nl = 0.f, sl = 0.f;
   float4 hu = make_float4(0.f, 0.f, 0.f, 0.f);
   float4 lu = hu, la = hu, nu = hu, su = hu;
-#pragma unroll (LATE ? 4 : RPT)
+#pragma unroll
   for (int j = 0; j < RPT; ++j) {
     const int r = rg + RG * j;   // < 16 * RG <= 512
     const int rr = r < kTailMaxK ? r : 0;

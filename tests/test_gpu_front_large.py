@@ -60,8 +60,8 @@ def _alone(kv, r):
 
 
 @pytest.mark.parametrize("requests,hq,hkv,b,d,longest,sp,topk,dtype,bounds", [
-    (9, 16, 2, 32, 64, 300, 57, 24, BF, "keys"),      # 18 rows, not dealt; odd slots
-    (16, 40, 8, 32, 128, 200, 13, 16, HF, "fp32"),    # five heads per KV head, dealt
+    (9, 16, 2, 32, 64, 300, 121, 24, BF, "keys"),     # 18 rows, not dealt; odd slots
+    (16, 40, 8, 32, 128, 200, 27, 16, HF, "fp32"),    # five heads per KV head, dealt
     (5, 8, 8, 32, 128, 2200, 4, 64, BF, "keys"),      # many chunks, two per workgroup
     (33, 8, 8, 16, 256, 500, 2, 8, BF, "fp32"),       # four chunks per workgroup, D = 256
     (9, 64, 8, 16, 128, 90, 31, 20, BF, "keys"),      # eight heads per KV head
