@@ -122,21 +122,30 @@ __global__ __launch_bounds__(256) void k_bounds(BoundsArgs a) {
 // streams its column down the block's B token rows, 16 loads of 16 bytes in
 // flight, and writes its 8 dims of lo and hi with two 16-byte stores each: no
 // LDS and no barrier.  One wave instruction reads 256-byte row segments of
-// 64 / (D / 8) consecutive blocks.  (Measured on c3's K, 151 MB: 30 us; the
-// one-block-per-workgroup layout below folds its token groups through LDS
-// with 8-way bank conflicts, 37 us.)
-#ifndef STK_BOUNDS_WG
-#define STK_BOUNDS_WG 64
-#endif
-#ifndef STK_BOUNDS_UNR
-#define STK_BOUNDS_UNR 16
-#endif
-template <typename T>
-__global__ __launch_bounds__(STK_BOUNDS_WG) void k_bounds_cols(BoundsArgs a) {
-  const int cpr = a.d / 8;
-  const int64_t gt = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// 64 / (D / 8) consecutive blocks.  The minimum and maximum are the CDNA4
+// three-operand ones that propagate NaN (v_minimum3_f32, v_maximum3_f32): two
+// rows per instruction, where comparing and selecting took nine VALU
+// instructions per key.
+//
+// STREAM: keys that do not stay in the 256 MB Infinity Cache are read with the
+// nontemporal hint, each XCD a contiguous range: 512 MB of bf16 keys (8 KV
+// heads x 7813 blocks x 32 x 128) 105.8 -> 103.4 us by the instructions, 90.4
+// with the hint (6.0 TB/s); 230 MB 42.2 -> 38.6.  Smaller keys are partly
+// there from the prefill that wrote them, and the hint costs more than it
+// saves: 134 MB 26.5 us without, 28.6 with.
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+constexpr int kColsWg = 64;
+constexpr int64_t kColsStream = 192ll << 20;
+constexpr int kColsUnr = 16;
+template <typename T, bool STREAM>
+__global__ __launch_bounds__(kColsWg) void k_bounds_cols(BoundsArgs a) {
+  const uint32_t cpr = a.d / 8;
+  const int wg = STREAM ? xcd_remap(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+  const int64_t gt = (int64_t)wg * kColsWg + threadIdx.x;
   if (gt >= (int64_t)a.rows * cpr) return;
-  const int row = (int)(gt / cpr), c = (int)(gt % cpr);
+  const bool narrow = (uint64_t)a.rows * cpr <= 0xffffffffull;   // 32-bit division
+  const int row = narrow ? (int)((uint32_t)gt / cpr) : (int)(gt / cpr);
+  const int c = (int)(gt - (int64_t)row * cpr);
   const T* base = reinterpret_cast<const T*>(a.k) + (size_t)row * a.b * a.d + 8 * c;
   float lo[8], hi[8];
 #pragma unroll
@@ -144,22 +153,25 @@ __global__ __launch_bounds__(STK_BOUNDS_WG) void k_bounds_cols(BoundsArgs a) {
     lo[e] = INFINITY;
     hi[e] = -INFINITY;
   }
-  constexpr int U = STK_BOUNDS_UNR;
+  constexpr int U = kColsUnr;
   for (int t0 = 0; t0 < a.b; t0 += U) {
     uint4 x[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int t = t0 + u < a.b ? t0 + u : t0;   // past B: token t0 again
-      x[u] = *reinterpret_cast<const uint4*>(base + (size_t)t * a.d);
+      const u32x4* p = reinterpret_cast<const u32x4*>(base + (size_t)t * a.d);
+      const u32x4 w = STREAM ? __builtin_nontemporal_load(p) : *p;
+      x[u] = make_uint4(w[0], w[1], w[2], w[3]);
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      float f[8];
+    for (int u = 0; u < U; u += 2) {
+      float f[8], g[8];
       unpack8<T>(x[u], f);
+      unpack8<T>(x[u + 1], g);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        lo[e] = nmin(lo[e], f[e]);
-        hi[e] = nmax(hi[e], f[e]);
+        lo[e] = __builtin_elementwise_minimum(__builtin_elementwise_minimum(lo[e], f[e]), g[e]);
+        hi[e] = __builtin_elementwise_maximum(__builtin_elementwise_maximum(hi[e], f[e]), g[e]);
       }
     }
   }
@@ -297,12 +309,19 @@ STK_API int stk_block_bounds(const void* k, int dtype, int hkv, int n, int b, in
   const bool vec16 = vec && ((reinterpret_cast<uintptr_t>(lo) | reinterpret_cast<uintptr_t>(hi)) &
                              15) == 0;
   const int64_t threads = (int64_t)a.rows * (d / 8);
-  const bool cols = vec16 && (threads + STK_BOUNDS_WG - 1) / STK_BOUNDS_WG <= 0x7fffffff;
-  const dim3 cgrid((unsigned)((threads + STK_BOUNDS_WG - 1) / STK_BOUNDS_WG));
+  const bool cols = vec16 && (threads + kColsWg - 1) / kColsWg <= 0x7fffffff;
+  const bool stream_keys = threads * b * 16 >= kColsStream;
+  const dim3 cgrid((unsigned)((threads + kColsWg - 1) / kColsWg));
   if (cols && dtype == DT_BF16) {
-    hipLaunchKernelGGL(k_bounds_cols<bf16s>, cgrid, dim3(STK_BOUNDS_WG), 0, st, a);
+    if (stream_keys)
+      hipLaunchKernelGGL((k_bounds_cols<bf16s, true>), cgrid, dim3(kColsWg), 0, st, a);
+    else
+      hipLaunchKernelGGL((k_bounds_cols<bf16s, false>), cgrid, dim3(kColsWg), 0, st, a);
   } else if (cols) {
-    hipLaunchKernelGGL(k_bounds_cols<f16s>, cgrid, dim3(STK_BOUNDS_WG), 0, st, a);
+    if (stream_keys)
+      hipLaunchKernelGGL((k_bounds_cols<f16s, true>), cgrid, dim3(kColsWg), 0, st, a);
+    else
+      hipLaunchKernelGGL((k_bounds_cols<f16s, false>), cgrid, dim3(kColsWg), 0, st, a);
   } else if (vec && dtype == DT_BF16)
     hipLaunchKernelGGL(k_bounds<bf16s>, dim3(a.rows), dim3(256), 0, st, a);
   else if (vec)
