@@ -7,6 +7,8 @@
 //   strict_topk/fused.py:10-220                     repair_fused
 //   strict_topk/gqa.py:62-104,384-413               repair_saved / repair_union
 //   strict_topk/gqa_light.py:10-92                  repair_saved_light / auto
+// The split and fused repairs run k_srepair (srepair_kernel.hpp) where it covers
+// the shape and the kernels here otherwise.
 // Every kernel here runs one workgroup (4 waves) per query head.  KV blocks
 // are read through the wave Tile routine; per-block states through weighted
 // LDS reductions.  Query head h reads KV head h / (Hq / Hkv).

@@ -55,7 +55,9 @@ def _signed(q, k, v, selected, predicted, prediction, min_remaining, cancellatio
 
 def repair_signed(q, k, v, selected, predicted, prediction, min_remaining=1.e-3,
                   cancellation_tol=1.e-5, max_extra_mass=0.):
-    """Signed repair in four launches (schedule, corrections, merge, fallback).
+    """Signed repair: schedule, corrections, merge and fallback, in the one launch
+    of ``signed_fused.repair_signed_fused`` where it covers the shape, else in
+    four.
 
     Each head's job list holds its missed selected blocks, then its wrong
     low blocks; one kernel computes every job's state.  The merge removes
