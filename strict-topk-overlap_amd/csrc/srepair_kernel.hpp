@@ -266,11 +266,14 @@ __global__ __launch_bounds__(kTailThreads) void k_srepair(SRepairArgs a) {
     const float pm = s_pm[rr], pl = s_pl[rr];
     const float wk = kp ? wexp(pm, mk) : 0.f;
     const float wn = wr ? wexp(pm, lm) : 0.f;
-    const float4 u4 = uu[j];
-    hl += wk * pl;
-    nl += wn * pl;
-    hu.x += wk * u4.x; hu.y += wk * u4.y; hu.z += wk * u4.z; hu.w += wk * u4.w;
-    nu.x += wn * u4.x; nu.y += wn * u4.y; nu.z += wn * u4.z; nu.w += wn * u4.w;
+    // a row that a sum does not take adds nothing to it, whatever it holds:
+    // taken by selection, as zero times NaN or an infinity is NaN
+    const float4 none = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 uk = kp ? uu[j] : none, un = wr ? uu[j] : none;
+    hl += wk * (kp ? pl : 0.f);
+    nl += wn * (wr ? pl : 0.f);
+    hu.x += wk * uk.x; hu.y += wk * uk.y; hu.z += wk * uk.z; hu.w += wk * uk.w;
+    nu.x += wn * un.x; nu.y += wn * un.y; nu.z += wn * un.z; nu.w += wn * un.w;
   }
 #pragma unroll
   for (int off = TPR; off < STK_WAVE; off <<= 1) {

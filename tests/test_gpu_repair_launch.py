@@ -91,3 +91,71 @@ def test_fallback_streams_tiles_when_a_state_is_not_finite():
             assert got.fallback.all()
             m = C.error_metrics(C.f64(got.output), want)
             assert m["passed"], (mode, fn.__name__, m)
+
+
+REPAIRS = ("split", "fused", "signed", "signed_fused")
+
+
+def _repair(name):
+    from strict_topk import fused, kernels, signed_fused, signed_repair
+    return {"split": (kernels.repair, O.repair), "fused": (fused.repair_fused, O.repair_fused),
+            "signed": (signed_repair.repair_signed, O.repair_signed),
+            "signed_fused": (signed_fused.repair_signed_fused, O.repair_signed_fused)}[name]
+
+
+def _check(name, ins, pred, opred, min_rem, tol, eps):
+    """One repair against the oracle's on the same prediction."""
+    q, k, v, a, p = ins
+    gpu, ref = _repair(name)
+    more = () if name == "split" else (eps,)
+    want = ref(C.f64(q), C.f64(k), C.f64(v), a.numpy(), p.numpy(), opred, min_rem, tol, *more)
+    got = gpu(*(t.to(DEV) for t in ins), pred, min_rem, tol, *more)
+    what = (name, pred.mode, eps)
+    assert got.fallback.cpu().numpy().tolist() == want.fallback.tolist(), what
+    np.testing.assert_allclose(got.remaining.cpu().double().numpy(), want.remaining, rtol=1e-4,
+                               atol=1e-6, err_msg=str(what))
+    if more and eps > 0:
+        assert got.approximate_heads.cpu().numpy().tolist() == want.approximate_heads.tolist()
+        np.testing.assert_allclose(got.extra_mass_bound.cpu().double().numpy(),
+                                   want.extra_mass_bound, rtol=1e-4, atol=1e-7)
+    m = C.error_metrics(C.f64(got.output), want.output)
+    assert m["passed"], (what, m)
+    return want
+
+
+@pytest.mark.parametrize("mode", ["saved", "hybrid", "compact"])
+@pytest.mark.parametrize("d,b,sp,slot", [
+    (128, 32, 24, 0),      # row 0, which rows past SP repeat
+    (128, 32, 24, 17),
+    (64, 16, 200, 130),    # sixteen row passes
+    (256, 32, 40, 0),
+])
+def test_rows_that_are_not_kept_add_nothing(d, b, sp, slot, mode):
+    """A predicted block that is not selected may hold anything: with NaN and an
+    infinity among its values the repairs give what the oracle gives, with the
+    oracle's flags."""
+    from strict_topk.kernels import speculate
+    h = 4
+    q, k, v, a, p = _inputs(h, h, 260, b, d, 24, sp, 0.7, BF, torch.int32)
+    for i in range(h):
+        chosen = set(a[i].tolist())
+        wrong = [j for j in range(sp) if int(p[i, j]) not in chosen]
+        j = wrong[0] if slot == 0 else min(wrong, key=lambda x: abs(x - slot))
+        if slot == 0:
+            p[i, [0, j]] = p[i, [j, 0]]
+            j = 0
+        v[i, int(p[i, j]), 3, 7] = float("inf") if i % 2 else float("nan")
+        v[i, int(p[i, j]), 1, 9] = float("-inf")
+    ins = (q, k, v, a, p)
+    for tau in (0.0, 0.05):
+        pred = speculate(*(t.to(DEV) for t in (q, k, v, p)), mode=mode, mass_threshold=tau,
+                         keep_mass=True)
+        opred = _oracle_pred(pred)
+        if mode == "compact":
+            opred.retained_ids = pred.retained_ids.cpu().numpy()
+        for name in REPAIRS:
+            with np.errstate(invalid="ignore"):
+                want = _check(name, ins, pred, opred, 1e-3, 1e-5, 0.01 if mode != "saved" else 0.0)
+            assert np.isfinite(want.output).all()
+            if tau == 0.0:
+                assert not want.fallback.any()
