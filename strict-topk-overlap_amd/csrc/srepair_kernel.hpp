@@ -47,10 +47,11 @@
 //      state (and a compact prediction's wrong blocks into a sum in the low
 //      frame);
 //   4. one merge by D threads and the guard flags OR-ed through LDS.  A
-//      flagged head's strict softmax over the selected blocks merges the
-//      states at hand (hits from the prediction's rows, misses from the
-//      waves), and a compact prediction's low hits are the only tiles read
-//      for it; if that is not finite, every selected tile is streamed again.
+//      flagged head's strict softmax over the selected blocks comes from their
+//      tiles alone: the misses' states, already formed, and the other selected
+//      slots' tiles, read now.  (Taking the hits from the prediction's rows
+//      saves those reads but counts a block predicted twice twice, and an
+//      altered state would pass the guard into the strict output.)
 // What bounds it is the chain of two memory round trips on one CU per head,
 // and that CU's tile rate (about 65 GB/s, 0.25 us per 16 KiB tile; two tiles
 // in flight in the fallback measured no faster than one).  At 16 heads x 48
@@ -86,7 +87,7 @@ __global__ __launch_bounds__(kTailThreads) void k_srepair(SRepairArgs a) {
   __shared__ uint8_t s_hi[kTailMaxK], s_hit[kTailMaxK], s_keep[kTailMaxK];
   __shared__ int jobs[COMPACT ? 2 * kTailMaxK : kTailMaxK];
   __shared__ int s_scan[kTailWaves];
-  __shared__ int s_bad, s_redo;
+  __shared__ int s_bad;
   __shared__ float s_hl[kTailWaves], s_nl[kTailWaves], s_wm[kTailWaves], s_wl[kTailWaves];
   __shared__ __align__(16) float s_hu[kTailWaves][D];
   __shared__ __align__(16) float s_nu[kTailWaves][D];
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(kTailThreads) void k_srepair(SRepairArgs a) {
     s_mm[tid] = mmv;
     s_ml[tid] = mlv;
   }
-  if (tid == 0) s_bad = s_redo = 0;
+  if (tid == 0) s_bad = 0;
   __syncthreads();
   // ---- membership (signed_repair.py:27-30): P[p] in A, A[a] not in P
   const bool amap = tid < sa && aid >= 0 && aid < nmap;
@@ -411,116 +412,41 @@ __global__ __launch_bounds__(kTailThreads) void k_srepair(SRepairArgs a) {
     return;
   }
   // ---- strict fallback (signed_fused.py:123-142): the softmax over the
-  // selected blocks from their states: the kept sums above, the misses'
-  // (s_wm, s_wl, s_wu, both still in LDS) and the low hits', which are
-  // prediction rows (read again) or, for a compact prediction, tiles
+  // selected blocks from their tiles alone, whatever the prediction holds.  The
+  // misses' states are at hand (s_wm, s_wl, s_wu); the other selected slots'
+  // tiles are read here, each slot once, wave w taking listed slots w, w + 8, ...
+  // (reads of s_scan, s_pm, s_nl, s_nu and jobs ended before the barrier above)
+  const bool rest = tid < sa && !miss;
+  int nrest;
+  const int at = block_excl_scan1(rest ? 1 : 0, s_scan, &nrest);
+  if (rest) jobs[at] = aid >= 0 && aid < n ? (int)aid : -1;
+  __syncthreads();
   float fm = -INFINITY, fz = 0.f, facc[TT::ACC];
 #pragma unroll
   for (int e = 0; e < TT::ACC; ++e) facc[e] = 0.f;
-  auto stream = [&](int64_t id) {
-    if (id < 0 || id >= n) return;
-    const size_t off = (((size_t)kvh * n + (size_t)id) * b) * D;
+  for (int x = w; x < nrest; x += kTailWaves) {
+    if (jobs[x] < 0) continue;
     for (int t0 = 0; t0 < b; t0 += TT::CH) {
-      t.load(K + off, V + off, t0, kw, vw);
+      t.load(K + tile(x), V + tile(x), t0, kw, vw);
       t.update(qw, kw, vw, t0, b, scale, fm, fz, facc);
     }
-  };
-  // (reads of s_nl, s_nu and jobs ended before the barrier above)
-  if constexpr (COMPACT) {
-    // selected blocks that are neither misses nor retained, in slot order
-    if (rmap) map_p[rid] = 2;
-    __syncthreads();
-    bool lowsel = false;
-    if (tid < sa && !miss) {
-      if (amap) {
-        lowsel = map_p[aid] != 2;
-      } else {
-        lowsel = true;
-        for (int j = 0; j < sc; ++j)
-          if (load_id(a.rids, a.ptype, (int64_t)h * sc + j) == aid) lowsel = false;
-      }
-    }
-    int nlow;
-    const int at = block_excl_scan1(lowsel ? 1 : 0, s_scan, &nlow);
-    if (lowsel) jobs[at] = tid;
-    __syncthreads();
-    for (int x = w; x < nlow; x += kTailWaves) stream(s_a[jobs[x]]);
-    if (lane_id() == 0) {
-      s_pm[w] = fm;
-      s_nl[w] = fz;
-    }
-    t.store(s_nu[w], facc);
-  } else {
-    // the low hits' rows relative to the waves' own maxima
-    float hm = -INFINITY, zl = 0.f;
-    float4 zu = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int r = rg; r < sp; r += RG)
-      if (s_hit[r] && !s_keep[r]) hm = fmaxf(hm, s_pm[r]);
-    hm = wave_max_u(hm);
-    for (int r = rg; r < sp; r += RG) {
-      if (!(s_hit[r] && !s_keep[r])) continue;
-      const float wt = wexp(s_pm[r], hm);
-      const float4 u4 =
-          *reinterpret_cast<const float4*>(a.pu + ((int64_t)h * sp + r) * D + 4 * c4);
-      zl += wt * s_pl[r];
-      zu.x += wt * u4.x; zu.y += wt * u4.y; zu.z += wt * u4.z; zu.w += wt * u4.w;
-    }
-#pragma unroll
-    for (int off = TPR; off < STK_WAVE; off <<= 1) {
-      zl += __shfl_xor(zl, off);
-      zu.x += __shfl_xor(zu.x, off); zu.y += __shfl_xor(zu.y, off);
-      zu.z += __shfl_xor(zu.z, off); zu.w += __shfl_xor(zu.w, off);
-    }
-    if (lane_id() < TPR) *reinterpret_cast<float4*>(&s_nu[w][4 * c4]) = zu;
-    __syncthreads();   // every wave has read s_pm
-    if (lane_id() == 0) {
-      s_pm[w] = hm;
-      s_nl[w] = zl;
-    }
   }
-  __syncthreads();
-  if (tid < D) {
-    float M = mk;
-#pragma unroll
-    for (int g = 0; g < kTailWaves; ++g) M = fmaxf(M, fmaxf(s_wm[g], s_pm[g]));
-    const float fk = wexp(mk, M);
-    float den = 0.f, num = 0.f;
-#pragma unroll
-    for (int g = 0; g < kTailWaves; ++g) {
-      const float f = wexp(s_wm[g], M), fn = wexp(s_pm[g], M);
-      den += fk * s_hl[g] + f * s_wl[g] + fn * s_nl[g];
-      num += fk * s_hu[g][tid] + f * s_wu[g][tid] + fn * s_nu[g][tid];
-    }
-    o = num / den;
-    if (is_bad(o)) s_redo = 1;
-  }
-  __syncthreads();
-  if (!s_redo) {
-    if (tid < D) a.out[(size_t)h * D + tid] = o;
-    return;
-  }
-  // not finite: every selected slot's tile, wave w taking slots w, w + 8, ...
-  fm = -INFINITY;
-  fz = 0.f;
-#pragma unroll
-  for (int e = 0; e < TT::ACC; ++e) facc[e] = 0.f;
-  for (int x = w; x < sa; x += kTailWaves) stream(s_a[x]);
   if (lane_id() == 0) {
-    s_wm[w] = fm;
-    s_wl[w] = fz;
+    s_pm[w] = fm;
+    s_nl[w] = fz;
   }
-  t.store(s_wu[w], facc);
+  t.store(s_nu[w], facc);
   __syncthreads();
   if (tid < D) {
     float M = -INFINITY;
 #pragma unroll
-    for (int g = 0; g < kTailWaves; ++g) M = fmaxf(M, s_wm[g]);
+    for (int g = 0; g < kTailWaves; ++g) M = fmaxf(M, fmaxf(s_wm[g], s_pm[g]));
     float den = 0.f, num = 0.f;
 #pragma unroll
     for (int g = 0; g < kTailWaves; ++g) {
-      const float f = wexp(s_wm[g], M);
-      den += f * s_wl[g];
-      num += f * s_wu[g][tid];
+      const float f = wexp(s_wm[g], M), fn = wexp(s_pm[g], M);
+      den += f * s_wl[g] + fn * s_nl[g];
+      num += f * s_wu[g][tid] + fn * s_nu[g][tid];
     }
     a.out[(size_t)h * D + tid] = num / den;
   }

@@ -159,3 +159,35 @@ def test_rows_that_are_not_kept_add_nothing(d, b, sp, slot, mode):
             assert np.isfinite(want.output).all()
             if tau == 0.0:
                 assert not want.fallback.any()
+
+
+@pytest.mark.parametrize("mode", ["hybrid", "compact"])
+@pytest.mark.parametrize("d,b,idtype", [(128, 32, torch.int32), (64, 64, torch.int64),
+                                        (256, 16, torch.int32)])
+def test_fallback_is_the_selected_blocks_alone(d, b, idtype, mode):
+    """A flagged head's output comes from the selected blocks, each slot once:
+    neither a block predicted twice nor a prediction whose kept states are no
+    longer those of the query changes it."""
+    from strict_topk.kernels import speculate
+    h, n, sa, sp = 4, 9000 if d == 64 else 120, 40, 40
+    q, k, v, a, p = _inputs(h, h, n, b, d, sa, sp, 0.7, BF, idtype)
+    for i in range(h):
+        # a selected block predicted twice (and an invalid selected ID below)
+        hits = [j for j in range(sp) if (a[i] == p[i, j]).any()]
+        p[i, hits[1]] = p[i, hits[0]]
+    a[:, -1] = -1
+    ins = (q, k, v, a, p)
+    exact = O.attention(C.f64(q), C.f64(k), C.f64(v), a[:, :-1].numpy())
+    for stale in (False, True):
+        pred = speculate(*(t.to(DEV) for t in (q, k, v, p)), mode=mode, mass_threshold=0.02,
+                         keep_mass=True)
+        if stale:
+            pred.state.u.mul_(-1.5)
+            pred.state.m.add_(0.25)
+        for name in REPAIRS:
+            # every fraction is below it
+            got = _repair(name)[0](*(t.to(DEV) for t in ins), pred, 2.0, 1e-5)
+            assert got.fallback.any()
+            flagged = got.fallback.cpu().numpy()
+            m = C.error_metrics(C.f64(got.output)[flagged], exact[flagged])
+            assert m["passed"], (name, mode, stale, m)
