@@ -4,7 +4,7 @@ Usage: python strict-topk-overlap_amd/build_lib.py [--jobs N]
 
 Objects go to strict-topk-overlap_amd/_build/, the shared library and the native
 host module next to the Python package (strict_topk/libstrict_topk_hip.so,
-strict_topk/_host.so), so they travel with the source tree.
+strict_topk/_host.<python tag>.so), so they travel with the source tree.
 """
 from __future__ import annotations
 
@@ -20,7 +20,7 @@ from pathlib import Path
 ROOT = Path(__file__).resolve().parent
 CSRC = ROOT / "csrc"
 OUT = ROOT / "strict_topk" / "libstrict_topk_hip.so"
-HOST = ROOT / "strict_topk" / "_host.so"
+HOST = ROOT / "strict_topk" / ("_host" + sysconfig.get_config_var("EXT_SUFFIX"))
 BUILD = ROOT / "_build"
 ARCH = "gfx950"
 SOURCES = ["api.cpp", "states.hip", "select.hip", "repair.hip", "signed.hip", "hier.hip", "sstep.hip",
@@ -77,6 +77,7 @@ def build_host() -> Path:
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall",
            "-Wno-sign-compare", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f'-DSTK_TORCH_VERSION="{torch.__version__}"',
            f"-isystem{root / 'include'}",
            f"-isystem{root / 'include' / 'torch' / 'csrc' / 'api' / 'include'}",
            "-isystem/opt/rocm/include", f"-isystem{sysconfig.get_path('include')}",
@@ -86,6 +87,8 @@ def build_host() -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"host module failed:\n{res.stderr}")
     os.replace(tmp, HOST)
+    # a module without the tag would be loaded by any Python
+    (HOST.parent / "_host.so").unlink(missing_ok=True)
     return HOST
 
 

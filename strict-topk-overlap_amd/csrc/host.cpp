@@ -318,4 +318,12 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, kMethods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host(void) { return PyModule_Create(&kModule); }
+// torch_version: the torch that the module was built for
+PyMODINIT_FUNC PyInit__host(void) {
+  PyObject* m = PyModule_Create(&kModule);
+  if (m && PyModule_AddStringConstant(m, "torch_version", STK_TORCH_VERSION)) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

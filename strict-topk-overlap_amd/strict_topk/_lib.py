@@ -9,8 +9,10 @@ a missing or unloadable library raises immediately.
 from __future__ import annotations
 
 import ctypes
+import importlib
 import os
 import threading
+import warnings
 from pathlib import Path
 
 import torch
@@ -117,20 +119,36 @@ def lib():
 _host = None
 
 
+class _PythonOnly:
+    """Stands in for the native host module where it cannot be used: every call
+    is left to the Python code, which checks and runs all of them."""
+
+    def speculative_step(self, *args):
+        return None
+
+    paged_step = prepared = speculative_step
+
+
 def host():
     """The native host path of the fused steps (csrc/host.cpp): its functions
-    return None for calls that the Python code has to check or refuse."""
+    return None for calls that the Python code has to check or refuse.  The
+    module is built for one Python and one torch; without one for this process
+    the steps run through the Python code alone, whose results are the same."""
     global _host
     if _host is None:
         handle = lib()
         try:
-            from . import _host as module
+            module = importlib.import_module("._host", __package__)
+            if module.torch_version != torch.__version__:
+                raise ImportError(f"built for torch {module.torch_version}")
+            module.bind(*(ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in (
+                "stk_step_supported", "stk_step_workspace_bytes", "stk_speculative_step",
+                "stk_paged_workspace_bytes", "stk_paged_step", "stk_paged_signed_step")))
         except ImportError as e:
-            raise RuntimeError("strict_topk native host module not built (run `python "
-                               "strict-topk-overlap_amd/build_lib.py`)") from e
-        module.bind(*(ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in (
-            "stk_step_supported", "stk_step_workspace_bytes", "stk_speculative_step",
-            "stk_paged_workspace_bytes", "stk_paged_step", "stk_paged_signed_step")))
+            warnings.warn(f"strict_topk native host module not used ({e}): the fused steps cost "
+                          "more host time; build it with `python strict-topk-overlap_amd/"
+                          "build_lib.py`", RuntimeWarning, stacklevel=2)
+            module = _PythonOnly()
         _host = module
     return _host
 

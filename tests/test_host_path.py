@@ -47,6 +47,27 @@ def test_declines_what_is_not_a_plain_gpu_call():
     assert host.speculative_step(nested, *a[1:], 8, False) is None
 
 
+@pytest.mark.parametrize("why", ["missing", "other torch"])
+def test_without_the_module_the_python_code_runs(monkeypatch, why):
+    """A process that cannot use the native module (none built for its Python, or
+    one built for another torch) keeps the Python path, and its refusals."""
+    import sys
+    import types
+
+    from strict_topk import _lib, step
+    name = "strict_topk._host"
+    monkeypatch.setattr(_lib, "_host", None)
+    monkeypatch.setitem(sys.modules, name, None if why == "missing" else
+                        types.SimpleNamespace(torch_version="0.0"))
+    with pytest.warns(RuntimeWarning, match="host module not used"):
+        host = _lib.host()
+    assert host.speculative_step(*_dense(), 8, False) is None
+    assert host.paged_step(*[None] * 15) is None and host.prepared(0) is None
+    assert _lib.host() is host                                     # warned once
+    with pytest.raises(ValueError, match="CUDA device"):
+        step.speculative_step(*_dense(), 8)
+
+
 @pytest.mark.gpu
 def test_step_equals_the_python_path(monkeypatch):
     from strict_topk import _lib, step
