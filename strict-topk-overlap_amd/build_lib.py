@@ -11,10 +11,12 @@ from __future__ import annotations
 import argparse
 import concurrent.futures as cf
 import os
+import re
 import shutil
 import subprocess
 import sys
 import sysconfig
+import tempfile
 from pathlib import Path
 
 ROOT = Path(__file__).resolve().parent
@@ -57,15 +59,62 @@ def _compile(src: str) -> Path:
     if _up_to_date(src, obj):
         return obj
     lang = ["-x", "hip"] if src.endswith(".hip") else []
-    cmd = [hipcc(), *FLAGS, *lang, "-c", str(CSRC / src), "-o", str(obj)]
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    noise = "packed-fp32-ops"
-    err = "\n".join(l for l in res.stderr.splitlines() if noise not in l)
-    if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed for {src}:\n{err}")
+    with tempfile.TemporaryDirectory(dir=BUILD) as tmp:
+        out = Path(tmp) / obj.name
+        keep = ["-save-temps=obj"] if lang else []
+        cmd = [hipcc(), *FLAGS, *keep, *lang, "-c", str(CSRC / src), "-o", str(out)]
+        res = subprocess.run(cmd, capture_output=True, text=True)
+        noise = "packed-fp32-ops"
+        err = "\n".join(l for l in res.stderr.splitlines() if noise not in l)
+        if res.returncode != 0:
+            raise RuntimeError(f"hipcc failed for {src}:\n{err}")
+        for asm in Path(tmp).glob(f"*-{ARCH}.s"):
+            bad = misplaced_copies(asm.read_text().splitlines())
+            if bad:
+                raise RuntimeError(f"{src}: register copies ahead of an exec restore (wrong "
+                                   "values in lanes that skip the branch); change the kernel's "
+                                   "register layout:\n" + "\n".join(bad))
+        os.replace(out, obj)
     if err.strip():
         sys.stderr.write(err + "\n")
     return obj
+
+
+def misplaced_copies(lines) -> list[str]:
+    """Places in gfx950 assembly where the compiler copies, spills or reloads a
+    vector register at the head of a join block, ahead of the instruction that
+    gives the lanes that skipped the branch their exec bits back: in those lanes
+    the copy is not made.  (Seen in a kernel that fills the register file: the
+    allocator put its copy before scalar copies that it had put before the
+    restore.  The sums of a wave whose rows were all skipped went to a wrong LDS
+    address.)"""
+    joins = {m[1] for l in lines if (m := re.match(r"\s+s_cbranch_execz (\S+)", l))}
+    block = re.compile(r"(\.LBB\d+_\d+):|; %bb\.\d+:")
+    copy = re.compile(r"(v_mov_b(32|64)_e32 v\S+ v|v_accvgpr_|scratch_(load|store)_)")
+    bad, pending, watch, fn, last = [], [], False, "", ""
+    for i, line in enumerate(lines, 1):
+        if m := block.match(line):
+            # a block without a label joins what it follows, unless a branch to
+            # the join just skipped it: then it is the branch's body
+            watch = m[1] in joins if m[1] else not last.startswith("s_cbranch_exec")
+            pending = []
+            continue
+        text = line.split(";")[0].strip()
+        if m := re.match(r"(_Z\w+):", text):
+            fn, watch = m[1], False
+        if not text or text.startswith("."):
+            continue
+        last = text
+        if not watch:
+            continue
+        if text.startswith("s_or_b64 exec, exec, "):
+            bad += [f"{fn} line {n}: {t}" for n, t in pending]
+            watch = False
+        elif re.match(r"s_\w+ exec,|s_\w+saveexec|s_c?branch", text):
+            watch = False
+        elif copy.match(text):
+            pending.append((i, text))
+    return bad
 
 
 def build_host() -> Path:

@@ -74,9 +74,12 @@ __device__ __forceinline__ void stail_head(const STailArgs& a) {
   constexpr int SW = kTailMaxK / STK_WAVE;   // slot words of wave 0
   // two tile buffers in flight when they fit the register budget
   constexpr bool DB = ONE && RPT == 4 && UP * TT::QW + 4 * TT::NV <= 64;
-  // the u rows are held from entry where the registers allow it; sixteen of
-  // them beside a D = 256 tile do not fit (with B = 16 the spilling build
-  // gave wrong sums for rows past SP): those are read where they are summed
+  // the u rows are held from entry where the registers allow it.  Sixteen of
+  // them beside a D = 256 tile fill the register file, and at B = 16 the
+  // compiler then put a copy of the lanes' LDS offset ahead of the exec restore
+  // of "r < sp": waves whose last row was past SP stored their sums to a wrong
+  // address (build_lib.py refuses such code).  Those rows are read where they
+  // are summed.
   constexpr bool LATE = NCH == 8 && RPT == 16;
   __shared__ int map[kTailMapN];
   __shared__ int sel[kTailMaxK], miss[kTailMaxK], pids[kTailMaxK];

@@ -147,3 +147,46 @@ def test_tails_at_row_and_key_edges(d, sp, n):
     for x, y in ((sg.result.output, want.output), (sg.result.output, gqa.exact(q, k, v, ids)),
                  (sg.result.remaining, want.remaining)):
         torch.testing.assert_close(x, y, rtol=3e-4, atol=3e-4)
+
+
+@pytest.mark.parametrize("dtype", [BF, HF])
+@pytest.mark.parametrize("d,sp,n", [
+    (128, 128, 300), (128, 129, 300), (128, 256, 300), (128, 200, 3000), (128, 256, 5000),
+    (256, 32, 200), (256, 33, 200), (256, 64, 200), (256, 65, 200), (256, 100, 200),
+    (256, 128, 200), (256, 65, 3000), (256, 33, 5000), (256, 127, 5000),
+])
+def test_tails_of_32_token_blocks_at_row_edges(d, sp, n, dtype):
+    """The tails whose tile is 32 tokens, dense and paged, at the edges of their
+    predicted-row passes and key counts, SP short of a whole pass among them:
+    outputs are those of the separate calls."""
+    from strict_topk import gqa, kernels, paged, signed_fused, step
+    hq, hkv, b, topk = 10, 2, 32, 37
+    gen = torch.Generator(device=DEV).manual_seed(d + sp + n)
+    q = torch.randn((hq, d), generator=gen, device=DEV, dtype=dtype)
+    k = torch.randn((hkv, n, b, d), generator=gen, device=DEV, dtype=dtype)
+    v = torch.randn((hkv, n, b, d), generator=gen, device=DEV, dtype=dtype)
+    lo, hi = k.amin(2), k.amax(2)
+    ids = gqa.select_blocks(q, lo.float(), hi.float(), topk)
+    noise = torch.rand((hq, n), generator=gen, device=DEV)
+    noise.scatter_(1, ids[:, : topk * 2 // 3].long(), 2.0)      # two thirds predicted
+    p = noise.topk(sp, dim=1).indices.to(torch.int32).contiguous()
+    want = gqa.exact(q, k, v, ids)
+    kv = paged.pack([(k, v)], bounds_dtype=dtype)
+    one = step.speculative_step(q, k, v, lo, hi, p, topk)
+    many = paged.speculative_step(q[None], kv, p[None], topk)
+    for sel, out in ((one.selected, one.output), (many.selected[0], many.output[0])):
+        assert torch.equal(sel, ids)
+        torch.testing.assert_close(out, want, rtol=3e-4, atol=3e-4)
+    for mode in ("saved", "hybrid"):
+        pred = kernels.speculate(q, k, v, p, mode, 0.02, keep_mass=True)
+        ref = signed_fused.repair_signed_fused(q, k, v, ids, p, pred)
+        sg = step.speculative_signed_step(q, k, v, lo, hi, p, topk, mode, 0.02)
+        pg = paged.speculative_signed_step(q[None], kv, p[None], topk, mode, 0.02)
+        for sel, res, at in ((sg.selected, sg.result, slice(None)), (pg.selected[0], pg.result, 0)):
+            assert torch.equal(sel, ids)
+            for x, y in ((res.output[at], want), (res.remaining[at], ref.remaining)):
+                torch.testing.assert_close(x, y, rtol=3e-4, atol=3e-4)
+            for x, y in ((res.total_jobs[at], ref.total_jobs),
+                         (res.positive_jobs[at], ref.positive_jobs),
+                         (res.fallback[at], ref.fallback)):
+                assert torch.equal(x, y)
