@@ -37,7 +37,7 @@ struct CompactStatesArgs {
 
 template <typename T, int NCH, int UP, typename I>
 __global__ __launch_bounds__(256, NCH <= 4 ? 4 : 2) void k_compact_states(CompactStatesArgs a) {
-  using TT = TokTile<T, NCH, UP>;
+  using TT = TokTile<T, NCH, UP, true>;
   const int wg = xcd_remap(blockIdx.x, gridDim.x);
   const int64_t item = (int64_t)wg * (blockDim.x / STK_WAVE) + wave_id();
   if (item >= (int64_t)a.hq * a.s) return;
