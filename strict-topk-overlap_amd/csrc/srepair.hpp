@@ -28,7 +28,12 @@ struct SRepairArgs {
 
 // Whether the one-launch kernel covers the shape: bf16 / fp16, D in
 // {64, 128, 256}, B a multiple of 16, SA, SP and SC <= 256, SC * D <= 32768,
-// 16-byte aligned q / k / v / state rows.
+// 16-byte aligned q / k / v / state rows.  It is the faster form over all of
+// it, the compact instances with B = 32 at D = 256 included, whose tiles and two
+// sums spill 400 to 470 bytes per lane: speculation and repair of 16 heads x 60
+// slots, four layers, 1306 us in the separate launches and 393 here (30 and 120
+// slots: 462 and 214, 2428 and 706; D = 128: 591 and 132; hybrid at D = 256: 299
+// and 137).
 bool srepair_covers(int dtype, int b, int d, int sa, int sp, int sc, uintptr_t align);
 
 int launch_srepair(int dtype, const SRepairArgs& a, hipStream_t st);

@@ -34,6 +34,16 @@ SHAPES = [
     (4, 1, 9000, 16, 64, 48, 48, 0.5, BF, 1.0, 0.0, 1e-3, 1e-5, torch.int64),     # past the maps
     (4, 4, 400, 32, 128, 256, 256, 0.9, BF, 0.008, 0.0, 1e-3, 1e-5, torch.int32), # widest rows
     (4, 4, 40, 32, 64, 1, 1, 0.0, BF, 0.1, 0.0, 1e-3, 1e-5, torch.int32),         # one row, missed
+    # D = 256 with low hits and wrong low blocks, whole-block tiles of 16 and 32
+    # tokens: compact rows of 26, 51 and 112 (four, eight and sixteen row passes)
+    (4, 2, 200, 32, 256, 40, 40, 0.6, BF, 0.04, 0.0, 1e-3, 1e-5, torch.int32),
+    (4, 2, 200, 32, 256, 60, 60, 0.5, HF, 0.02, 0.02, 1e-3, 1e-5, torch.int64),
+    (4, 2, 300, 32, 256, 70, 128, 0.6, BF, 0.009, 0.0, 1e-3, 1e-5, torch.int32),
+    (4, 2, 300, 32, 256, 70, 128, 0.6, HF, 0.009, 0.0, 1.0, 1e-5, torch.int32),   # all fall back
+    (4, 2, 200, 16, 256, 40, 40, 0.6, HF, 0.04, 0.0, 1e-3, 1e-5, torch.int32),
+    (4, 2, 200, 16, 256, 60, 60, 0.5, BF, 0.02, 0.0, 1.0, 1e-5, torch.int32),     # all fall back
+    (4, 2, 300, 16, 256, 70, 128, 0.6, BF, 0.009, 0.01, 1e-3, 1e-5, torch.int64),
+    (4, 4, 300, 32, 128, 64, 200, 0.6, BF, 0.006, 0.0, 1e-3, 1e-5, torch.int32),  # 167 rows
 ]
 
 
