@@ -55,11 +55,13 @@ __device__ __forceinline__ void states_tok_wg(const StatesArgs& a, int wg,
                                               const Paging& pg = Paging{}) {
   using TT = TokTile<T, NCH, UP>;
   const int waves = blockDim.x / STK_WAVE;
-  // (the states of 2^32 items would not fit the device: 32-bit divisions)
-  const uint32_t item32 = (uint32_t)wg * waves + __builtin_amdgcn_readfirstlane(wave_id());
-  if (item32 >= (uint64_t)a.hq * a.s) return;
-  const int64_t item = item32;
-  const int h = (int)(item32 / (uint32_t)a.s);
+  // (a 32-bit index through readfirstlane was slower: 155.0 -> 155.5 us for
+  // twelve one-launch steps of 16 heads x 512 blocks, 18.9 -> 19.2 and 42.3 ->
+  // 42.6 for paged batches of 2 and 8 requests, 173.4 -> 174.7 for eight steps
+  // at D = 256)
+  const int64_t item = (int64_t)wg * waves + wave_id();
+  if (item >= (int64_t)a.hq * a.s) return;
+  const int h = (int)(item / a.s);
   TT t;
   t.init();
   uint32_t qw[TT::QW];
