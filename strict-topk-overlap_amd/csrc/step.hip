@@ -76,21 +76,30 @@ FrontArgs make_front_args(const void* q, const void* k, const void* v, int dtype
   // with the next one's bounds in flight, and a paged states wave takes two
   // slots (its table reads once for both; a third round trip that the dense
   // wave does not have, where two slots were slower, 54.3 against 50.8 us at
-  // 64 heads x 96 slots x 8000 blocks).  Measured per step, single against
-  // multi: 24 ragged paged requests x 32 heads x 64 slots 174 -> 134 us; 8
-  // requests x 64 heads x 64 slots 63.2 -> 58.1.  With up to four query heads
-  // per KV head the middle sizes lose (32 heads, 8-16 requests of 200-500
-  // blocks, 10752-16384 slots, D = 128: 33.0 -> 33.5, 41.0 -> 42.0), so those
-  // stay single up to 24576 slots (12 requests x 32 heads x 53 slots, D = 256:
-  // 146 -> 121); dense grids gain 2 % from 2048 slots.
+  // 64 heads x 96 slots x 8000 blocks).  Measured per step, single against multi,
+  // by the predicted slots of a paged batch:
+  //   more than four query heads per KV head (64 heads x 64 slots, requests of 300
+  //   to 500 blocks): 4096 slots 18.0 -> 17.4 us, 8192 26.7 -> 25.7, 12288 33.0 ->
+  //   32.8, 16384 38.4 -> 38.0, 20480 and 24576 within 1 %, 32768 67.6 -> 66.0;
+  //   D = 256 (32 heads x 53 slots, 100 to 300 blocks): 3392 even, 6784 42.0 ->
+  //   40.2, 10176 54.5 -> 52.9, 13568 75.0 -> 71.1, 20352 122.1 -> 112.6;
+  //   up to four heads per KV head at D = 128 (32 heads x 64 slots, 100 to 400
+  //   blocks): 20480 even, 24576 53.6 -> 54.1, 28672 60.9 -> 61.0, 32768 74.3 ->
+  //   71.8, 49152 121.0 -> 115.4; with lengths of 40 to 1000 blocks 24576 58.1 ->
+  //   53.4; between 10752 and 16384 slots 33.0 -> 33.5 and 41.0 -> 42.0 at 200 to
+  //   500 blocks.
+  // Dense grids gain 2 % from 2048 slots.
   const int64_t least = !paged ? 2048 : (G > 4 || d > 128 ? 4096 : 24576);
   f.multi = s.one && G <= kFrontMultiG && (items >= least || chunks >= 2048);
   if (f.multi) {
-    // two slots per wave: 4096 slots 25.4 -> 26.1 us, 16384 slots 52.7 -> 50.8;
-    // 8192 slots beside 2048 chunks 41.6 -> 38.7
+    // two slots per wave: 4096 slots 25.4 -> 26.1 us, 16384 slots 52.7 -> 50.8
+    // (64 heads: 38.8 -> 37.8), 32768 71.0 -> 66.2; 8192 slots beside 2048 chunks
+    // 41.6 -> 38.7
     f.ipw = paged && items >= 8192 && (items >= 16384 || chunks >= 2048) ? 2 : 1;
-    // 4096 chunks: 1, 2, 4 per workgroup 104.9, 100.1, 103.6 us; 11656 (a ragged
-    // batch, mostly past its rows' ends): 29.9, 24.4, 21.2
+    // chunks per workgroup, 1 against 2 from 2048 chunks: 4096 chunks 30.7 -> 28.7
+    // us, 6144 38.5 -> 36.1; 2 against 4 from 8192: 8192 45.9 -> 45.2 and 37.2 ->
+    // 36.6 (two batches), 12288 68.6 -> 67.0, 16384 57.4 -> 54.3, 23312 103.7 ->
+    // 99.8
     f.cpw = chunks >= 8192 ? 4 : (chunks >= 2048 ? 2 : 1);
     f.score_wgs = (f.sc.chunks + f.cpw - 1) / f.cpw;
     f.total_wgs = f.score_wgs + (G * ((sp + f.ipw - 1) / f.ipw) + 3) / 4;
