@@ -118,11 +118,11 @@ __device__ __forceinline__ void repair_fast_head(const GqaRepairArgs& a, int h) 
   float4 hu = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (int j = 0; j < RPT; ++j) {
-    const int r = rg + RG * j;
     const float wt = used[j] ? wexp(um[j], hm) : 0.f;
-    // rows past sp were loaded from row 0: zero them
-    const float4 ur = r < sp ? uu[j] : make_float4(0.f, 0.f, 0.f, 0.f);
-    hl += wt * ul[j];
+    // a row that is not summed (past sp, not selected) adds nothing, whatever it
+    // holds: zero times NaN or an infinity would be NaN
+    const float4 ur = used[j] ? uu[j] : make_float4(0.f, 0.f, 0.f, 0.f);
+    hl += wt * (used[j] ? ul[j] : 0.f);
     hu.x += wt * ur.x; hu.y += wt * ur.y; hu.z += wt * ur.z; hu.w += wt * ur.w;
   }
   static_assert(TPR <= STK_WAVE, "state rows wider than a wave");

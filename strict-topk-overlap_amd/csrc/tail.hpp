@@ -225,11 +225,11 @@ __device__ __forceinline__ void tail_head(const TailArgs& a) {
   float4 hu = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
   for (int j = 0; j < RPT; ++j) {
-    const int r = rg + RG * j;
     const float wt = used[j] ? wexp(um[j], hm) : 0.f;
-    // rows past sp were loaded from row 0 (or a stand-in buffer): zero them
-    const float4 ur = r < sp ? uu[j] : make_float4(0.f, 0.f, 0.f, 0.f);
-    hl += wt * ul[j];
+    // a row that is not summed (past sp, not selected) adds nothing, whatever it
+    // holds: zero times NaN or an infinity would be NaN
+    const float4 ur = used[j] ? uu[j] : make_float4(0.f, 0.f, 0.f, 0.f);
+    hl += wt * (used[j] ? ul[j] : 0.f);
     hu.x += wt * ur.x; hu.y += wt * ur.y; hu.z += wt * ur.z; hu.w += wt * ur.w;
   }
   // fold the row groups of this wave (lanes with the same columns)

@@ -81,6 +81,7 @@ __device__ __forceinline__ void stail_head(const STailArgs& a) {
   // address (build_lib.py refuses such code).  Those rows are read where they
   // are summed.
   constexpr bool LATE = NCH == 8 && RPT == 16;
+  constexpr int UNR = LATE ? 4 : RPT;   // rows in flight in their sums
   __shared__ int map[kTailMapN];
   __shared__ int sel[kTailMaxK], miss[kTailMaxK], pids[kTailMaxK];
   __shared__ float s_pm[kTailMaxK], s_pl[kTailMaxK];
@@ -354,7 +355,7 @@ __device__ __forceinline__ void stail_head(const STailArgs& a) {
   float hl = 0.f, nl = 0.f, sl = 0.f;
   float4 hu = make_float4(0.f, 0.f, 0.f, 0.f);
   float4 lu = hu, la = hu, nu = hu, su = hu;
-#pragma unroll
+#pragma unroll UNR
   for (int j = 0; j < RPT; ++j) {
     const int r = rg + RG * j;   // < 16 * RG <= 512
     const int rr = r < kTailMaxK ? r : 0;
@@ -373,18 +374,23 @@ __device__ __forceinline__ void stail_head(const STailArgs& a) {
     const float wl = lo ? wexp(pm, lowm) : 0.f;
     const float wn = wr ? wl : 0.f;
     const float ws = us ? wexp(pm, mu) : 0.f;
-    // rows past sp were loaded from row 0 (or a stand-in buffer): zero them
+    // a row that a sum does not take (past sp, not selected, not low) adds
+    // nothing to it, whatever it holds: zero times NaN or an infinity would be
+    // NaN.  Selected rows go to hu and su, low ones to lu, la and nu.
     const float4 ux = LATE ? u_row(j) : uu[LATE ? 0 : j];
-    const float4 u4 = r < sp ? ux : make_float4(0.f, 0.f, 0.f, 0.f);
-    hl += wk * pl;
-    nl += wn * pl;
-    sl += ws * pl;
-    hu.x += wk * u4.x; hu.y += wk * u4.y; hu.z += wk * u4.z; hu.w += wk * u4.w;
-    lu.x += wl * u4.x; lu.y += wl * u4.y; lu.z += wl * u4.z; lu.w += wl * u4.w;
-    la.x += wl * fabsf(u4.x); la.y += wl * fabsf(u4.y);
-    la.z += wl * fabsf(u4.z); la.w += wl * fabsf(u4.w);
-    nu.x += wn * u4.x; nu.y += wn * u4.y; nu.z += wn * u4.z; nu.w += wn * u4.w;
-    su.x += ws * u4.x; su.y += ws * u4.y; su.z += ws * u4.z; su.w += ws * u4.w;
+    const float4 none = make_float4(0.f, 0.f, 0.f, 0.f);
+    const bool ht = kp || us;
+    const float4 uh = ht ? ux : none, ul = lo ? ux : none;
+    const float ph = ht ? pl : 0.f;
+    hl += wk * ph;
+    nl += wn * (lo ? pl : 0.f);
+    sl += ws * ph;
+    hu.x += wk * uh.x; hu.y += wk * uh.y; hu.z += wk * uh.z; hu.w += wk * uh.w;
+    su.x += ws * uh.x; su.y += ws * uh.y; su.z += ws * uh.z; su.w += ws * uh.w;
+    lu.x += wl * ul.x; lu.y += wl * ul.y; lu.z += wl * ul.z; lu.w += wl * ul.w;
+    la.x += wl * fabsf(ul.x); la.y += wl * fabsf(ul.y);
+    la.z += wl * fabsf(ul.z); la.w += wl * fabsf(ul.w);
+    nu.x += wn * ul.x; nu.y += wn * ul.y; nu.z += wn * ul.z; nu.w += wn * ul.w;
   }
   // fold the row groups of this wave (lanes with the same columns)
 #pragma unroll
