@@ -79,8 +79,11 @@ __device__ __forceinline__ void stail_head(const STailArgs& a) {
   // compiler then put a copy of the lanes' LDS offset ahead of the exec restore
   // of "r < sp": waves whose last row was past SP stored their sums to a wrong
   // address (build_lib.py refuses such code).  Those rows are read where they
-  // are summed.
-  constexpr bool LATE = NCH == 8 && RPT == 16;
+  // are summed, four at a time: 4 requests x 32 heads of 500 to 900 blocks, 100
+  // slots, D = 256, 125.6 -> 114.1 us at B = 32 and 71.5 -> 70.3 at B = 16; 200
+  // slots at D = 128, B = 32 101.9 -> 90.7.  Held rows stay the faster form with
+  // eight passes (D = 256, B = 32, 60 slots: 84.3 against 86.0).
+  constexpr bool LATE = RPT == 16 && (NCH == 8 || (NCH == 4 && UP == 2));
   constexpr int UNR = LATE ? 4 : RPT;   // rows in flight in their sums
   __shared__ int map[kTailMapN];
   __shared__ int sel[kTailMaxK], miss[kTailMaxK], pids[kTailMaxK];
