@@ -55,10 +55,11 @@
 // What bounds it is the chain of two memory round trips on one CU per head,
 // and that CU's tile rate (about 65 GB/s, 0.25 us per 16 KiB tile; two tiles
 // in flight in the fallback measured no faster than one).  At 16 heads x 48
-// slots of 32 x 128 bf16, hybrid, a quarter missed: 9.6 us, where the
+// slots of 32 x 128 bf16, hybrid, a quarter missed: 9.2 us, where the
 // four-wave k_repair_fused took 55.3; at 32 heads x 64 slots fp16, compact, a
-// fifth missed and some head flagged: 21 us, where k_membership,
-// k_states_tok, k_wrong_aggregate, k_hybrid_merge and k_fallback took 117.
+// fifth missed: 13.6 us, 21.6 with a flagged head, whose other selected tiles
+// come through one CU, where k_membership, k_states_tok, k_wrong_aggregate,
+// k_hybrid_merge and k_fallback took 117.
 // Results agree with the separate launches up to FP32 reduction order.
 #pragma once
 
