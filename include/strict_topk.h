@@ -132,6 +132,13 @@ int stk_fallback(const void* q, const void* k, const void* v, int dtype, int hq,
                  int b, int d, const void* selected, int sel_dtype, int sa, const uint8_t* flags,
                  float* out, void* stream);
 
+/* 1 when stk_repair, stk_repair_fused and stk_repair_signed run as one launch
+ * for these shapes and operands (address_bits: the addresses of q, k, v and the
+ * prediction's u, OR-ed): stk_repair and stk_repair_signed then need no
+ * workspace and take a null one. */
+int stk_repair_one_launch(int dtype, int b, int d, int sa, int sp, int sc, int mode,
+                          size_t address_bits);
+
 size_t stk_repair_workspace_bytes(int hq, int sa, int sp, int sc, int d, int mode);
 
 /* strict_topk/kernels.py:504-550 repair (split path: membership, miss

@@ -418,6 +418,12 @@ STK_API int stk_fallback(const void* q, const void* k, const void* v, int dtype,
   return stk_check_launch("k_fallback");
 }
 
+STK_API int stk_repair_one_launch(int dtype, int b, int d, int sa, int sp, int sc, int mode,
+                                  size_t address_bits) {
+  return (mode == MODE_COMPACT || sc == sp) &&
+         srepair_covers(dtype, b, d, sa, sp, sc, (uintptr_t)address_bits);
+}
+
 STK_API size_t stk_repair_workspace_bytes(int hq, int sa, int sp, int sc, int d, int mode) {
   size_t b = 0;
   b += stk_align((size_t)hq * sc);            // hit
@@ -449,12 +455,10 @@ STK_API int stk_repair(const void* q, const void* k, const void* v, int dtype, i
   STK_REQUIRE(mode == MODE_SAVED || (high && low_m && low_l && low_u && low_abs), "null low group");
   STK_REQUIRE(mode != MODE_COMPACT || retained_ids, "null retained ids");
   STK_REQUIRE(sc > 0 && sc <= kMaxIds, "bad prediction state width");
-  STK_REQUIRE(workspace && workspace_bytes >= stk_repair_workspace_bytes(hq, sa, sp, sc, d, mode),
-              "workspace too small");
   hipStream_t st = (hipStream_t)stream;
   const uintptr_t align = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
                           reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(pu);
-  if ((mode == MODE_COMPACT || sc == sp) && srepair_covers(dtype, b, d, sa, sp, sc, align)) {
+  if (stk_repair_one_launch(dtype, b, d, sa, sp, sc, mode, align)) {
     SRepairArgs r{{q, k, v, hq, hkv, n, b, d}, selected, sel_dtype, sa, predicted, pred_dtype, sp,
                   mode != MODE_SAVED ? 1 : 0, sc, mode == MODE_COMPACT ? retained_ids : nullptr, 1,
                   pm, pl, pu, high, low_m, low_l, low_u, low_abs, nullptr, nullptr, min_remaining,
@@ -462,6 +466,8 @@ STK_API int stk_repair(const void* q, const void* k, const void* v, int dtype, i
                   nullptr, nullptr};
     return launch_srepair(dtype, r, st);
   }
+  STK_REQUIRE(workspace && workspace_bytes >= stk_repair_workspace_bytes(hq, sa, sp, sc, d, mode),
+              "workspace too small");
   Carve w(workspace);
   uint8_t* hit = w.take<uint8_t>((size_t)hq * sc);
   uint8_t* miss = w.take<uint8_t>((size_t)hq * sa);
@@ -540,7 +546,7 @@ STK_API int stk_repair_fused(const void* q, const void* k, const void* v, int dt
   hipStream_t st = (hipStream_t)stream;
   const uintptr_t align = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
                           reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(pu);
-  if ((mode == MODE_COMPACT || sc == sp) && srepair_covers(dtype, b, d, sa, sp, sc, align)) {
+  if (stk_repair_one_launch(dtype, b, d, sa, sp, sc, mode, align)) {
     SRepairArgs r{{q, k, v, hq, hkv, n, b, d}, selected, sel_dtype, sa, predicted, pred_dtype, sp,
                   mode != MODE_SAVED ? 1 : 0, sc, mode == MODE_COMPACT ? retained_ids : nullptr, 0,
                   pm, pl, pu, high, low_m, low_l, low_u, low_abs, mass_m, mass_l, min_remaining,

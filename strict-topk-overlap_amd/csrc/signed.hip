@@ -326,13 +326,11 @@ STK_API int stk_repair_signed(const void* q, const void* k, const void* v, int d
   STK_REQUIRE(max_extra_mass == 0.f || (approximate && extra_mass_bound), "null budget outputs");
   STK_REQUIRE(max_extra_mass == 0.f || mode == MODE_SAVED || (mass_m && mass_l),
               "positive max_extra_mass requires speculate(..., keep_mass=True)");
-  STK_REQUIRE(workspace && workspace_bytes >= stk_signed_workspace_bytes(hq, sa, sp, sc, d, mode),
-              "workspace too small");
   hipStream_t st = (hipStream_t)stream;
   int cap = mode == MODE_SAVED ? sa : sa + sp;
   const uintptr_t align = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
                           reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(pu);
-  if ((mode == MODE_COMPACT || sc == sp) && srepair_covers(dtype, b, d, sa, sp, sc, align)) {
+  if (stk_repair_one_launch(dtype, b, d, sa, sp, sc, mode, align)) {
     // one launch: schedule, corrections and guarded merge (srepair_kernel.hpp)
     SRepairArgs r{{q, k, v, hq, hkv, n, b, d}, selected, sel_dtype, sa, predicted, pred_dtype, sp,
                   mode != MODE_SAVED ? 1 : 0, sc, mode == MODE_COMPACT ? retained_ids : nullptr, 0,
@@ -342,6 +340,8 @@ STK_API int stk_repair_signed(const void* q, const void* k, const void* v, int d
                   approximate, extra_mass_bound};
     return launch_srepair(dtype, r, st);
   }
+  STK_REQUIRE(workspace && workspace_bytes >= stk_signed_workspace_bytes(hq, sa, sp, sc, d, mode),
+              "workspace too small");
   Carve w(workspace);
   uint8_t* keep = w.take<uint8_t>((size_t)hq * sc);
   uint8_t* low_hit = w.take<uint8_t>((size_t)hq);

@@ -44,6 +44,7 @@ _SIGS = {
                                   P, P, P, P, P, P, P, P, P, P, P, P, P, Z, P]),
     "stk_touch_kv": (I, [P, P, I, I, I, I, I, P, I, I, P, P]),
     "stk_fallback": (I, [P, P, P, I, I, I, I, I, I, P, I, I, P, P, P]),
+    "stk_repair_one_launch": (I, [I, I, I, I, I, I, I, Z]),
     "stk_repair_workspace_bytes": (Z, [I, I, I, I, I, I]),
     "stk_repair": (I, [P, P, P, I, I, I, I, I, I, P, I, I, P, I, I, I, I,
                        P, P, P, P, P, P, P, P, P, F, F, P, P, P, P, Z, P]),

@@ -191,6 +191,18 @@ def prediction_args(prediction, q):
             _lib.ptr(prediction.retained_ids if prediction.mode == 'compact' else None))
 
 
+def repair_workspace(query, q, k, v, prediction, sa, sp):
+    """Scratch memory of a repair's separate launches (size by ``query``), or
+    None where the repair is one launch and needs none."""
+    u = prediction.state.u
+    b, d = k.shape[2:]
+    mode, sc = MODES[prediction.mode], u.shape[1]
+    bits = q.data_ptr() | k.data_ptr() | v.data_ptr() | u.data_ptr()
+    if _lib.size("stk_repair_one_launch", _lib.dtype_code(q), b, d, sa, sp, sc, mode, bits):
+        return None
+    return _lib.workspace(_lib.size(query, q.shape[0], sa, sp, sc, d, mode), q.device)
+
+
 def repair(q, k, v, selected, predicted, prediction, min_remaining=1.e-3, cancellation_tol=1.e-5):
     """Bring a prediction back to the exact output over the selected set.
 
@@ -205,15 +217,14 @@ def repair(q, k, v, selected, predicted, prediction, min_remaining=1.e-3, cancel
     h, n, b, d, sa = _shape(q, k, v, selected)
     sp = predicted.shape[1]
     pa = prediction_args(prediction, q)
-    mode, sc = pa[0], pa[1]
     out = torch.empty((h, d), device=q.device, dtype=torch.float32)
     fallback = torch.empty((h,), device=q.device, dtype=torch.bool)
     remaining = torch.empty((h,), device=q.device, dtype=torch.float32)
-    ws = _lib.workspace(_lib.size("stk_repair_workspace_bytes", h, sa, sp, sc, d, mode), q.device)
+    ws = repair_workspace("stk_repair_workspace_bytes", q, k, v, prediction, sa, sp)
     _lib.call("stk_repair", *_args(q, k, v), _lib.ptr(selected), _lib.id_code(selected), sa,
               _lib.ptr(predicted), _lib.id_code(predicted), sp, *pa, float(min_remaining),
               float(cancellation_tol), _lib.ptr(out), _lib.ptr(fallback), _lib.ptr(remaining),
-              _lib.ptr(ws), ws.numel(), _lib.stream(q.device))
+              _lib.ptr(ws), 0 if ws is None else ws.numel(), _lib.stream(q.device))
     return RepairResult(out, fallback, remaining)
 
 

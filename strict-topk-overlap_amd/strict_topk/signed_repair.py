@@ -11,7 +11,7 @@ from dataclasses import dataclass
 import torch
 
 from . import _lib
-from .kernels import RepairResult, _args, _shape, prediction_args
+from .kernels import RepairResult, _args, _shape, prediction_args, repair_workspace
 
 
 @dataclass
@@ -30,7 +30,6 @@ def _signed(q, k, v, selected, predicted, prediction, min_remaining, cancellatio
     if hybrid and max_extra_mass > 0 and (prediction.mass_m is None or prediction.mass_l is None):
         raise ValueError("positive max_extra_mass requires speculate(..., keep_mass=True)")
     pa = prediction_args(prediction, q)
-    mode, sc = pa[0], pa[1]
     capacity = sa + sp if hybrid else sa
     dev = q.device
     id_dtype = torch.promote_types(selected.dtype, predicted.dtype)
@@ -42,14 +41,14 @@ def _signed(q, k, v, selected, predicted, prediction, min_remaining, cancellatio
     remaining = torch.empty((h,), device=dev, dtype=torch.float32)
     approximate = torch.empty_like(fallback) if max_extra_mass > 0 else None
     extra = torch.empty_like(remaining) if max_extra_mass > 0 else None
-    ws = _lib.workspace(_lib.size("stk_signed_workspace_bytes", h, sa, sp, sc, d, mode), dev)
+    ws = repair_workspace("stk_signed_workspace_bytes", q, k, v, prediction, sa, sp)
     _lib.call("stk_repair_signed", *_args(q, k, v), _lib.ptr(selected), _lib.id_code(selected), sa,
               _lib.ptr(predicted), _lib.id_code(predicted), sp, *pa, _lib.ptr(prediction.mass_m),
               _lib.ptr(prediction.mass_l), float(min_remaining), float(cancellation_tol),
               float(max_extra_mass), 1 if fused else 0, _lib.ptr(queue), _lib.id_code(queue),
               _lib.ptr(positive), _lib.ptr(total), _lib.ptr(out), _lib.ptr(fallback),
               _lib.ptr(remaining), _lib.ptr(approximate), _lib.ptr(extra), _lib.ptr(ws),
-              ws.numel(), _lib.stream(dev))
+              0 if ws is None else ws.numel(), _lib.stream(dev))
     return SignedRepairResult(out, fallback, remaining, approximate, extra, positive, total)
 
 

@@ -133,3 +133,27 @@ def test_documented_binding_matches_header():
     assert any(kind == "call" for _, kind, _ in found)
     wrong = [(name, kind, n, decls.get(name)) for name, kind, n in found if decls.get(name) != n]
     assert not wrong, wrong
+
+
+def test_one_launch_repairs_need_no_workspace(lib):
+    """stk_repair_one_launch names the shapes whose repairs are one launch, and only
+    the others ask for a workspace (checked before any device is touched)."""
+    L = lib.lib()
+    saved, hybrid, compact = 0, 1, 2
+    assert L.stk_repair_one_launch(2, 32, 128, 64, 64, 64, hybrid, 1 << 20) == 1
+    assert L.stk_repair_one_launch(1, 16, 256, 64, 128, 40, compact, 0) == 1
+    for args in ((0, 32, 128, 64, 64, 64, hybrid, 0),       # fp32
+                 (2, 8, 128, 64, 64, 64, saved, 0),         # blocks of 8
+                 (2, 32, 96, 64, 64, 64, saved, 0),         # D = 96
+                 (2, 32, 128, 257, 64, 64, saved, 0),       # more than 256 selected
+                 (2, 32, 256, 64, 129, 129, hybrid, 0),     # SC * D past 32768
+                 (2, 32, 128, 64, 64, 40, hybrid, 0),       # a state row per slot, but compact
+                 (2, 32, 128, 64, 64, 64, hybrid, 8)):      # an operand off 16 bytes
+        assert L.stk_repair_one_launch(*args) == 0, args
+    x = 4096                                                # any address: nothing is read
+    head = [x, x, x, 0, 4, 4, 10, 32, 128, x, 0, 8, x, 0, 8, saved, 8, x, x, x] + [None] * 6
+    assert L.stk_repair(*head, 1e-3, 1e-5, x, x, x, None, 0, None) == -1
+    assert b"workspace too small" in L.stk_last_error()
+    assert L.stk_repair_signed(*head, None, None, 1e-3, 1e-5, 0.0, 1, x, 0, x, x, x, x, x, None,
+                               None, None, 0, None) == -1
+    assert b"workspace too small" in L.stk_last_error()
